@@ -82,11 +82,10 @@ template <int D, int NWV>
 struct Gemm1Shared {
     static_assert(NWV == 4 || NWV == 8, "waves per workgroup");
     static constexpr int kSlot = 32 * kBlk;                 // a wave's weight transpose slot
-    static constexpr int kTokStage = 64 * kBlk + 64 * 4;    // 64 token rows + their scales
+    static constexpr int kTokStage = 64 * kBlk + 2 * 64 * 4;   // 64 token rows, their scales, zeros
     static constexpr int kStages = D + 1;
     static constexpr int kLds = NWV * kSlot + kStages * kTokStage;
     static constexpr int kItems = kI / (16 * NWV);          // work items per tile
-    static constexpr int kRowsPerWave = 64 / NWV;           // token rows each wave moves
 };
 
 // One item of gemm1_shared_kernel with CB live 16-row blocks (the tile has 16 CB - 15 ..
@@ -126,23 +125,26 @@ __device__ __forceinline__ void gemm1_shared_item(
     // the NWV groups of a workgroup lie in one 128-column scale block
     const float* sg = s1 + (size_t)(le * kN1B + (ng >> 3)) * kHB;
     const float* su = sg + (size_t)kIB * kHB;
-    // token rows of this wave, 8 per instruction (clamped into the tile), for the live
-    // blocks: the stage rows of a live block are always written, so no stale row
-    // reaches an MFMA
-    constexpr int NT = S::kRowsPerWave / 8;
-    bool tlive[NT];
+    // token rows of the live blocks (16 CB stage rows, 8 per instruction, clamped into the
+    // tile), spread over the waves: wave w moves rows 8 (w + NWV i) ...  Every wave issues
+    // the same number of loads per K block whatever is live, so that the number of loads in
+    // flight is known at compile time: the loads it has no rows (or, but for wave 0, no
+    // scales) for get an offset past the buffer, which moves nothing.
+    constexpr int NT = (2 * CB + NWV - 1) / NWV;
+    constexpr uint32_t kNothing = 0xfffffff0u;
     uint32_t toff[NT];
-    int ntok = 0;
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
-        const int tr = S::kRowsPerWave * wave + 8 * i + drow;
-        tlive[i] = S::kRowsPerWave * wave + 8 * i < 16 * CB;
-        toff[i] = (uint32_t)sorted_tok[row0 + min(tr, nrows - 1)] * kH + ((dchunk ^ swz128(tr)) << 4);
-        ntok += tlive[i] ? 1 : 0;
+        const int q = wave + NWV * i;
+        const int tr = 8 * q + drow;
+        const uint32_t o = (uint32_t)sorted_tok[row0 + min(tr, nrows - 1)] * kH + ((dchunk ^ swz128(tr)) << 4);
+        toff[i] = q < 2 * CB ? o : kNothing;
     }
     const int sr = min(lane, nrows - 1);
-    const uint32_t soff = (uint32_t)(sa.by_row ? row0 + sr : sorted_tok[row0 + sr]) * 4;
-    const int nvm = 4 + ntok + (wave == 0 ? 1 : 0);   // loads per K block
+    const uint32_t so = (uint32_t)(sa.by_row ? row0 + sr : sorted_tok[row0 + sr]) * 4;
+    const uint32_t soff = wave == 0 ? so : kNothing;
+    const int sdst = 64 * kBlk + (wave == 0 ? 0 : 64 * 4);   // the others' zeros land past the scales
+    constexpr int kVm = 4 + NT + 1;                          // loads per wave and K block
 
     // K block kb: weights in ring slot kb % D, token rows in stage kb % (D + 1)
     v4u bw[D][4];
@@ -153,8 +155,8 @@ __device__ __forceinline__ void gemm1_shared_item(
         uint8_t* st = tok0 + (kb % S::kStages) * S::kTokStage;
 #pragma unroll
         for (int i = 0; i < NT; ++i)
-            if (tlive[i]) bdma16(rs_h, toff[i], (uint32_t)kb * kBlk, st + (S::kRowsPerWave * wave + 8 * i) * kBlk);
-        if (wave == 0) bdma4(rs_s, soff, (uint32_t)kb * sa.stride * 4, st + 64 * kBlk);
+            bdma16(rs_h, toff[i], (uint32_t)kb * kBlk, st + 8 * (wave + NWV * i) * kBlk);
+        bdma4(rs_s, soff, (uint32_t)kb * sa.stride * 4, st + sdst);
     };
 #pragma unroll
     for (int k = 0; k < D - 1; ++k) issue(k, k);
@@ -162,58 +164,73 @@ __device__ __forceinline__ void gemm1_shared_item(
     v4f ag[CB], au[CB];
 #pragma unroll
     for (int c = 0; c < CB; ++c) ag[c] = au[c] = zero;
+    // One K block, `younger` later blocks in flight.  The loads are unconditional and the
+    // last blocks peeled because the wait before a ring slot's use is counted by the
+    // compiler too, as the fewest loads any path issues after it: with the token loads
+    // under a wave's own branch and the last blocks' loads skipped in the loop, that count
+    // was 0 in every second K block, which drained the ring there.  With three workgroups per
+    // CU the others covered that (GEMM1 unchanged, 132 registers instead of 153); the
+    // token-sharing GEMM2, at two per CU, gained 9% from the same change.
+    auto block = [&](int kb, int j, auto younger) {
+        // this wave's loads of block kb are in (those of the blocks after it may stay in
+        // flight); after the barrier, every wave's (the token stage)
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(decltype(younger)::value * kVm));
+        lds_barrier();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) *reinterpret_cast<v4u*>(slot + wr[i]) = bw[j][i];
+        const uint8_t* st = tok0 + (kb % S::kStages) * S::kTokStage;
+        const float* ssc = reinterpret_cast<const float*>(st + 64 * kBlk);
+        const float wg = sg[kb], wu = su[kb];
+        const v4u g0 = *reinterpret_cast<const v4u*>(slot + rd_g0);
+        const v4u g1 = *reinterpret_cast<const v4u*>(slot + rd_g1);
+        const v4u u0 = *reinterpret_cast<const v4u*>(slot + 16 * kBlk + rd_g0);
+        const v4u u1 = *reinterpret_cast<const v4u*>(slot + 16 * kBlk + rd_g1);
+        const v8i bg = {(int)g0[0], (int)g0[1], (int)g0[2], (int)g0[3], (int)g1[0], (int)g1[1], (int)g1[2], (int)g1[3]};
+        const v8i bu = {(int)u0[0], (int)u0[1], (int)u0[2], (int)u0[3], (int)u1[0], (int)u1[1], (int)u1[2], (int)u1[3]};
+#pragma unroll
+        for (int c = 0; c < CB; ++c) {
+            __builtin_amdgcn_sched_barrier(0);   // one row block at a time: short live ranges
+            const uint8_t* ts = st + 16 * c * kBlk;
+            const v4u a0 = *reinterpret_cast<const v4u*>(ts + rd_g0);
+            const v4u a1 = *reinterpret_cast<const v4u*>(ts + rd_g1);
+            const v8i ba = {(int)a0[0], (int)a0[1], (int)a0[2], (int)a0[3], (int)a1[0], (int)a1[1], (int)a1[2], (int)a1[3]};
+            const float sc = ssc[16 * c + r16];
+            const float fg = sc * wg, fu = sc * wu;
+            const v4f tg = mfma_fp8(bg, ba, zero);
+            const v4f tu = mfma_fp8(bu, ba, zero);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                ag[c][v] = __builtin_fmaf(tg[v], fg, ag[c][v]);
+                au[c][v] = __builtin_fmaf(tu[v], fu, au[c][v]);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
 #pragma unroll 1
-    for (int kb0 = 0; kb0 < kHB; kb0 += D) {
+    for (int kb0 = 0; kb0 < kHB - D; kb0 += D) {
 #pragma unroll
         for (int j = 0; j < D; ++j) {
-            const int kb = kb0 + j;
             // block kb + D - 1 goes to the ring slot block kb - 1 used (written to the LDS
             // slot before) and to the stage of block kb - 2, which every wave finished
             // reading before the barrier of block kb - 1
-            if (kb + D - 1 < kHB) issue(kb + D - 1, (j + D - 1) % D);
+            issue(kb0 + j + D - 1, (j + D - 1) % D);
             __builtin_amdgcn_sched_barrier(0);
-            // this wave's loads of block kb are in (those of the D - 1 blocks after it
-            // may stay in flight); after the barrier, every wave's (the token stage)
-            wait_vm_upto24(min(kHB - 1 - kb, D - 1) * nvm);
-            lds_barrier();
-#pragma unroll
-            for (int i = 0; i < 4; ++i) *reinterpret_cast<v4u*>(slot + wr[i]) = bw[j][i];
-            const uint8_t* st = tok0 + (kb % S::kStages) * S::kTokStage;
-            const float* ssc = reinterpret_cast<const float*>(st + 64 * kBlk);
-            const float wg = sg[kb], wu = su[kb];
-            const v4u g0 = *reinterpret_cast<const v4u*>(slot + rd_g0);
-            const v4u g1 = *reinterpret_cast<const v4u*>(slot + rd_g1);
-            const v4u u0 = *reinterpret_cast<const v4u*>(slot + 16 * kBlk + rd_g0);
-            const v4u u1 = *reinterpret_cast<const v4u*>(slot + 16 * kBlk + rd_g1);
-            const v8i bg = {(int)g0[0], (int)g0[1], (int)g0[2], (int)g0[3], (int)g1[0], (int)g1[1], (int)g1[2], (int)g1[3]};
-            const v8i bu = {(int)u0[0], (int)u0[1], (int)u0[2], (int)u0[3], (int)u1[0], (int)u1[1], (int)u1[2], (int)u1[3]};
-#pragma unroll
-            for (int c = 0; c < CB; ++c) {
-                __builtin_amdgcn_sched_barrier(0);   // one row block at a time: short live ranges
-                const uint8_t* ts = st + 16 * c * kBlk;
-                const v4u a0 = *reinterpret_cast<const v4u*>(ts + rd_g0);
-                const v4u a1 = *reinterpret_cast<const v4u*>(ts + rd_g1);
-                const v8i ba = {(int)a0[0], (int)a0[1], (int)a0[2], (int)a0[3], (int)a1[0], (int)a1[1], (int)a1[2], (int)a1[3]};
-                const float sc = ssc[16 * c + r16];
-                const float fg = sc * wg, fu = sc * wu;
-                const v4f tg = mfma_fp8(bg, ba, zero);
-                const v4f tu = mfma_fp8(bu, ba, zero);
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    ag[c][v] = __builtin_fmaf(tg[v], fg, ag[c][v]);
-                    au[c][v] = __builtin_fmaf(tu[v], fu, au[c][v]);
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
+            block(kb0 + j, j, IntC<D - 1>{});
         }
     }
+    issue(kHB - 1, D - 1);
+    __builtin_amdgcn_sched_barrier(0);
+    block(kHB - D, 0, IntC<D - 1>{});
+    [&]<int... J>(std::integer_sequence<int, J...>) {
+        (block(kHB - D + 1 + J, 1 + J, IntC<D - 2 - J>{}), ...);
+    }(std::make_integer_sequence<int, D - 1>{});
 #pragma unroll
     for (int c = 0; c < CB; ++c)
         store_swiglu4(C, c_wide, row0 + 16 * c + r16, ng * 16 + kq * 4, ag[c], au[c], 16 * c + r16 < nrows);
 }
 
 // WPE: the waves per SIMD the register allocation is held to (1: the compiler's choice,
-// 172 registers, two workgroups per CU; 3: 153 registers, three).
+// 164 registers; 3: 132 registers, three workgroups per CU).
 // With three per CU the kernel chooses, from the call's tile count, how many of its 768
 // workgroups work: items are equal (an item streams 128 weight rows over all of K), so the
 // rounds decide the time, and 768 < items <= 1024 takes two rounds either way, where two

@@ -15,13 +15,16 @@
 // in the streaming kernels), together with the K block's W2 scale (a vector load, so the
 // K loop issues no scalar load that an LDS access would wait for).  The tile's C rows of
 // a K block (64 rows x 256 bytes of fp16) come once for the whole workgroup by
-// buffer_load ... lds into a ring of D + 1 stages (wave w moves rows 16 w .. 16 w + 15;
-// a 16-row block past the tile moves nothing and its MFMAs are skipped); one barrier per
-// K block hands a stage over.  In a stage, row r keeps its 16-byte chunk c at position
+// buffer_load ... lds into a ring of D + 1 stages (the live 16-row blocks' loads spread
+// evenly over the waves; a block past the tile moves nothing and its MFMAs are skipped);
+// one barrier per K block hands a stage over.  Every wave issues the same loads in every K
+// block and the last blocks are peeled, so that the waits count exactly the loads in
+// flight; with loads under a wave's own branch the compiler's waits drained the W2 ring in
+// every second K block (24 experts of ~29 rows, T = 509: 90.7 -> 82.9 us).  In a stage, row r keeps its 16-byte chunk c at position
 // c ^ (r mod 16), so the 16 rows an MFMA operand read touches land on 16 different bank
 // groups.  It reads C in the fp16 form the token-sharing GEMM1 writes, so the fp16 ->
 // hi/lo conversion launch of the prefill GEMM2 goes away, and it has two workgroups per CU
-// (212 registers, 64 KB of LDS) where the prefill GEMM2 has one.  Measured against that
+// (204 registers, 64 KB of LDS) where the prefill GEMM2 has one.  Measured against that
 // pair it is faster while the tiles hold few rows (T = 200 .. 559, the plan there) and
 // slower beyond, where it moves about as much C per item as W2 at a similar per-CU rate.
 // When GEMM1 flagged C beyond the fp16 range, each wave computes its columns on the rare
@@ -80,18 +83,19 @@ __device__ __forceinline__ void gemm2_shared_item(
     }
     // the item's W2 scale block: one scale per K block for every wave
     const __amdgpu_buffer_rsrc_t rs_s = buffer_rsrc(s2 + (size_t)(le * kHB + (hg0 >> 3)) * kIB, kIB * 4);
-    // C rows 16 wave .. 16 wave + 15 of the tile (clamped into it), 4 rows per instruction:
-    // lane L moves row 4 i + L / 16 of them into stage chunk L % 16, which holds the row's
-    // chunk (L % 16) ^ (row % 16)
+    // C rows of the live blocks (clamped into the tile), 4 rows per instruction, the 4 CB
+    // instructions spread evenly over the waves: lane L of instruction wave + 4 i moves row
+    // 4 (wave + 4 i) + L / 16 into stage chunk L % 16, which holds the row's chunk
+    // (L % 16) ^ (row % 16)
     const __amdgpu_buffer_rsrc_t rs_c = buffer_rsrc(C.f16() + (size_t)row0 * kI, 64u * kI * 2);
-    const bool clive = 16 * wave < nrows;
-    uint32_t coff[4];
+    constexpr int NC = CB;
+    uint32_t coff[NC];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int r = 16 * wave + 4 * i + (lane >> 4);
+    for (int i = 0; i < NC; ++i) {
+        const int r = 4 * (wave + 4 * i) + (lane >> 4);
         coff[i] = (uint32_t)min(r, nrows - 1) * (kI * 2) + (uint32_t)(((lane & 15) ^ (r & 15)) << 4);
     }
-    const int nvm = 2 * HF + 1 + (clive ? 4 : 0);   // loads per K block
+    constexpr int kVm = 2 * HF + 1 + NC;         // loads per wave and K block
 
     // K block kb: W2 rows and scale in ring slot kb % D, C rows in stage kb % (D + 1)
     v4u bw[D][2 * HF];
@@ -102,10 +106,8 @@ __device__ __forceinline__ void gemm2_shared_item(
             bw[ring][i] = __builtin_amdgcn_raw_buffer_load_b128(rs_w, woff[i], (uint32_t)kb * kBlk, 2);
         bsc[ring] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs_s, 0u, (uint32_t)kb * 4, 0));
         uint8_t* st = cst0 + (kb % S::kStages) * S::kCStage;
-        if (clive) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) bdma16(rs_c, coff[i], (uint32_t)kb * S::kRow, st + (16 * wave + 4 * i) * S::kRow);
-        }
+        for (int i = 0; i < NC; ++i) bdma16(rs_c, coff[i], (uint32_t)kb * S::kRow, st + 4 * (wave + 4 * i) * S::kRow);
     };
 #pragma unroll
     for (int k = 0; k < D - 1; ++k) issue(k, k);
@@ -115,52 +117,60 @@ __device__ __forceinline__ void gemm2_shared_item(
     for (int hf = 0; hf < HF; ++hf)
 #pragma unroll
         for (int c = 0; c < CB; ++c) acc[hf][c] = zero;
+    auto block = [&](int kb, int j, auto younger) {
+        // this wave's loads of block kb are in (those of the blocks after it may stay in
+        // flight); after the barrier, every wave's (the C stage)
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(decltype(younger)::value * kVm));
+        lds_barrier();
+#pragma unroll
+        for (int i = 0; i < 2 * HF; ++i) *reinterpret_cast<v4u*>(slot + wr[i]) = bw[j][i];
+        uint32_t ww[HF][8];
+#pragma unroll
+        for (int hf = 0; hf < HF; ++hf) {
+            const v4u x0 = *reinterpret_cast<const v4u*>(slot + hf * 16 * kBlk + rd0);
+            const v4u x1 = *reinterpret_cast<const v4u*>(slot + hf * 16 * kBlk + rd1);
+            ww[hf][0] = x0[0]; ww[hf][1] = x0[1]; ww[hf][2] = x0[2]; ww[hf][3] = x0[3];
+            ww[hf][4] = x1[0]; ww[hf][5] = x1[1]; ww[hf][6] = x1[2]; ww[hf][7] = x1[3];
+        }
+        const uint8_t* st = cst0 + (kb % S::kStages) * S::kCStage;
+        const float sb = bsc[j];
+#pragma unroll
+        for (int c = 0; c < CB; ++c) {
+            __builtin_amdgcn_sched_barrier(0);   // one row block at a time: short live ranges
+            // C row 16 c + r16, elements 32 kq + 8 q .. + 7 of the K block for MFMA q
+            const uint8_t* crow = st + (16 * c + r16) * S::kRow;
+            v4u cf[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) cf[q] = *reinterpret_cast<const v4u*>(crow + (((4 * kq + q) ^ r16) << 4));
+#pragma unroll
+            for (int hf = 0; hf < HF; ++hf) {
+                v4f t = zero;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) t = mfma_w2_c<true>(ww[hf][2 * q], ww[hf][2 * q + 1], cf[q], t);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[hf][c][v] = __builtin_fmaf(t[v], sb, acc[hf][c][v]);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
 #pragma unroll 1
-    for (int kb0 = 0; kb0 < kIB; kb0 += D) {
+    for (int kb0 = 0; kb0 < kIB - D; kb0 += D) {
 #pragma unroll
         for (int j = 0; j < D; ++j) {
-            const int kb = kb0 + j;
             // block kb + D - 1 goes to the ring slot block kb - 1 used (written to the LDS
             // slot before) and to the stage of block kb - 2, which every wave finished
             // reading before the barrier of block kb - 1
-            if (kb + D - 1 < kIB) issue(kb + D - 1, (j + D - 1) % D);
+            issue(kb0 + j + D - 1, (j + D - 1) % D);
             __builtin_amdgcn_sched_barrier(0);
-            // this wave's loads of block kb are in (those of the D - 1 blocks after it may
-            // stay in flight); after the barrier, every wave's (the C stage)
-            wait_vm_upto24(min(kIB - 1 - kb, D - 1) * nvm);
-            lds_barrier();
-#pragma unroll
-            for (int i = 0; i < 2 * HF; ++i) *reinterpret_cast<v4u*>(slot + wr[i]) = bw[j][i];
-            uint32_t ww[HF][8];
-#pragma unroll
-            for (int hf = 0; hf < HF; ++hf) {
-                const v4u x0 = *reinterpret_cast<const v4u*>(slot + hf * 16 * kBlk + rd0);
-                const v4u x1 = *reinterpret_cast<const v4u*>(slot + hf * 16 * kBlk + rd1);
-                ww[hf][0] = x0[0]; ww[hf][1] = x0[1]; ww[hf][2] = x0[2]; ww[hf][3] = x0[3];
-                ww[hf][4] = x1[0]; ww[hf][5] = x1[1]; ww[hf][6] = x1[2]; ww[hf][7] = x1[3];
-            }
-            const uint8_t* st = cst0 + (kb % S::kStages) * S::kCStage;
-            const float sb = bsc[j];
-#pragma unroll
-            for (int c = 0; c < CB; ++c) {
-                __builtin_amdgcn_sched_barrier(0);   // one row block at a time: short live ranges
-                // C row 16 c + r16, elements 32 kq + 8 q .. + 7 of the K block for MFMA q
-                const uint8_t* crow = st + (16 * c + r16) * S::kRow;
-                v4u cf[4];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) cf[q] = *reinterpret_cast<const v4u*>(crow + (((4 * kq + q) ^ r16) << 4));
-#pragma unroll
-                for (int hf = 0; hf < HF; ++hf) {
-                    v4f t = zero;
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) t = mfma_w2_c<true>(ww[hf][2 * q], ww[hf][2 * q + 1], cf[q], t);
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) acc[hf][c][v] = __builtin_fmaf(t[v], sb, acc[hf][c][v]);
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
+            block(kb0 + j, j, IntC<D - 1>{});
         }
     }
+    issue(kIB - 1, D - 1);
+    __builtin_amdgcn_sched_barrier(0);
+    block(kIB - D, 0, IntC<D - 1>{});
+    [&]<int... J>(std::integer_sequence<int, J...>) {
+        (block(kIB - D + 1 + J, 1 + J, IntC<D - 2 - J>{}), ...);
+    }(std::make_integer_sequence<int, D - 1>{});
 #pragma unroll
     for (int c = 0; c < CB; ++c)
 #pragma unroll
