@@ -37,7 +37,7 @@ bool launch_dispatch_masks(const int*, const float*, const uint32_t*, int, int, 
                            hipStream_t);
 bool launch_gemm1(int, const uint8_t*, const TokenScales&, int, const uint8_t*, const float*,
                   const int4*, const int*, const int*, int, const int*, const Intermediate&,
-                  bool, hipStream_t);
+                  bool, bool, hipStream_t);
 bool launch_gemm1_dispatch(const RouteIn&, int*, float*, int, int, const uint8_t*, const float*,
                            const uint8_t*, const float*, int*, int4*, int*, float*, int*,
                            const Intermediate&, hipStream_t);
@@ -64,7 +64,6 @@ using moe::host::check_forward_args;
 using moe::host::clamp_offset;
 using moe::host::fill_layout;
 using moe::host::kMaxT;
-using moe::host::kRankedMaxT;
 using moe::host::Plan;
 using moe::host::workspace_regions;
 
@@ -160,7 +159,8 @@ int forward_impl(const moe_mi355_args& a, void* workspace, size_t ws_bytes, hipS
     // HIP call left in this thread's last-error slot is cleared first.
     (void)hipGetLastError();
     const bool prof = (a.flags & MOE_MI355_FLAG_PROFILE) && g_prof.rec && g_prof.used < g_prof.slots;
-    const bool ranked = !(a.flags & MOE_MI355_FLAG_LIST_ORDER) && T <= kRankedMaxT;
+    // the row-class GEMM1 has no 256-row tile list to take its items from
+    const bool ranked = plan.row_class || !(a.flags & MOE_MI355_FLAG_LIST_ORDER);
     moe::KernelTimer* timer = prof ? &g_prof.rec[g_prof.used++] : nullptr;
     if (timer) timer->n = 0;
     auto stage = [timer](int st) {
@@ -212,9 +212,9 @@ int forward_impl(const moe_mi355_args& a, void* workspace, size_t ws_bytes, hipS
                                               stok, sw, inv, inter, s);
     }
     else
-        ok = ok && moe::launch_gemm1(plan.g1, a.hidden_states, sa, T, a.gemm1_weights,
-                                     a.gemm1_weights_scale, tiles, num_tiles, meta, max_tiles,
-                                     stok, inter, ranked, s);
+        ok = ok && moe::launch_gemm1(plan.row_class ? 4 : plan.g1, a.hidden_states, sa, T,
+                                     a.gemm1_weights, a.gemm1_weights_scale, tiles, num_tiles, meta,
+                                     max_tiles, stok, inter, ranked, plan.row_class, s);
     stage(3);
     if (ok && plan.convert) moe::launch_c_f16_to_hilo(inter, meta, s);   // in the GEMM2 stage
     if (ok && plan.combine_in_gemm2)      // GEMM2 writes the output (timed as the GEMM2 stage)

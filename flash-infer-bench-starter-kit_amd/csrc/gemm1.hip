@@ -26,6 +26,7 @@
 #include "gemm1_stream.h"
 #include "route_token.h"
 
+#include <algorithm>
 #include <mutex>
 
 MOE_STAMP_TABLE(gemm1)
@@ -168,9 +169,7 @@ __device__ __forceinline__ void gemm1_shared_item(
     // last blocks peeled because the wait before a ring slot's use is counted by the
     // compiler too, as the fewest loads any path issues after it: with the token loads
     // under a wave's own branch and the last blocks' loads skipped in the loop, that count
-    // was 0 in every second K block, which drained the ring there.  With three workgroups per
-    // CU the others covered that (GEMM1 unchanged, 132 registers instead of 153); the
-    // token-sharing GEMM2, at two per CU, gained 9% from the same change.
+    // was 0 in every second K block, which drained the ring there (T = 509: GEMM1 143 us).
     auto block = [&](int kb, int j, auto younger) {
         // this wave's loads of block kb are in (those of the blocks after it may stay in
         // flight); after the barrier, every wave's (the token stage)
@@ -230,7 +229,7 @@ __device__ __forceinline__ void gemm1_shared_item(
 }
 
 // WPE: the waves per SIMD the register allocation is held to (1: the compiler's choice,
-// 164 registers; 3: 132 registers, three workgroups per CU).
+// 172 registers, two workgroups per CU; 3: 153 registers, three).
 // With three per CU the kernel chooses, from the call's tile count, how many of its 768
 // workgroups work: items are equal (an item streams 128 weight rows over all of K), so the
 // rounds decide the time, and 768 < items <= 1024 takes two rounds either way, where two
@@ -432,41 +431,42 @@ __global__ __launch_bounds__(NRW == 8 ? 512 : 256) void gemm1_rstream_dispatch_k
     MOE_STAMP(3 * (int)blockIdx.x + 2);
 }
 
-// Epilogue of the prefill GEMM1 kernels: SwiGLU, then the fp8 hi/lo form of C.
-// The wave holds 64 rows x 64 SwiGLU columns (acc[s][j]: j < 4 gate, j >= 4 up; lane
-// holds D[col 16j + 4kq + v][row 16s + r16]); its partner wave (wn ^ 1) holds the other
-// 64 columns of the 128-column block ng, so the row amax is combined across the two
-// through LDS (xch, 2 KB, reusing the operand ring: every wave must have left the
-// K loop, hence the first barrier).  Per row: s = amax/448 (1 for an all-zero row),
-// hi = e4m3(c * 448/amax), lo = e4m3((c - hi*s) * 16*448/amax).
-// A lane's 4 bytes of a row in each of the 4 column blocks are transposed across the
-// row's 4 lanes (lanes l, l+16, l+32, l+48) with v_permlane32_swap / v_permlane16_swap,
-// after which lane kq holds 16 consecutive bytes: one 16-byte store per form and row
-// block instead of four 4-byte ones, each row's 64 bytes written by one instruction.
-__device__ __forceinline__ void store_c_hilo(const v4f (&acc)[4][8], float* xch, int wm, int wn,
+// Epilogue of the prefill GEMM1: SwiGLU, then the fp8 hi/lo form of C.  The wave holds 128
+// rows x 32 SwiGLU columns (acc[s][i]: i < 2 gate, i >= 2 up; lane holds D[col 16 i + 4 kq
+// + v][row 16 s + r16]); the waves wn = 0 .. 3 hold the 128 columns of block ng, so the row
+// amax is combined across them through LDS (xch, [4][256] floats).  Per row: s = amax/448
+// (1 for an all-zero row), hi = e4m3(c * 448/amax), lo = e4m3((c - hi*s) * 16*448/amax).
+// A lane's 4 bytes of two rows in each of the 2 column blocks are transposed across the
+// rows' 4 lanes (lanes l, l+16, l+32, l+48) with v_permlane32_swap / v_permlane16_swap,
+// after which a lane holds 16 consecutive bytes of one row: one 16-byte store per form for
+// two row blocks.  Row blocks past the tile (from `live` on, uniform) are skipped.
+__device__ __forceinline__ void store_c_hilo(const v4f (&acc)[8][4], float* xch, int live, int wm, int wn,
                                              int kq, int r16, int row0, int nrows, int ng,
-                                             const Intermediate& C) {
-    float c[4][4][4];
-    float m[4];
+                                             const Intermediate& C, bool through_f16) {
+    float c[8][2][4];
+    float m[8];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
+    for (int s = 0; s < 8; ++s) {
+        if (s >= live) continue;
         m[s] = 0.f;
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                c[s][j][v] = silu_f32(acc[s][j + 4][v]) * acc[s][j][v];
-                m[s] = fmaxf(m[s], fabsf(c[s][j][v]));
+                float x = silu_f32(acc[s][i + 2][v]) * acc[s][i][v];
+                if (through_f16) {
+                    // the fp32 product first, then fp16 (fused into one rounding otherwise)
+                    __asm__ volatile("" : "+v"(x));
+                    if (fabsf(x) <= kF16Max) x = (float)(_Float16)x;
+                }
+                c[s][i][v] = x;
+                m[s] = fmaxf(m[s], fabsf(x));
             }
         m[s] = fmaxf(m[s], __shfl_xor(m[s], 16));
         m[s] = fmaxf(m[s], __shfl_xor(m[s], 32));
+        if (kq == 0) xch[wn * 256 + 128 * wm + 16 * s + r16] = m[s];
     }
-    __syncthreads();
-    if (kq == 0) {
-#pragma unroll
-        for (int s = 0; s < 4; ++s) xch[(wm * 2 + wn) * 64 + 16 * s + r16] = m[s];
-    }
-    __syncthreads();
+    lds_barrier();
     // 4 x 4 transpose of 32-bit words over the 16-lane rows of the wave (word j of row kq
     // -> word kq of row j): 32-lane then 16-lane swaps
     auto transpose4 = [](uint32_t (&w)[4]) {
@@ -480,104 +480,150 @@ __device__ __forceinline__ void store_c_hilo(const v4f (&acc)[4][8], float* xch,
         w[2] = p[0]; w[3] = p[1];
     };
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-        const float amax = fmaxf(m[s], xch[(wm * 2 + (wn ^ 1)) * 64 + 16 * s + r16]);
-        const int r = 64 * wm + 16 * s + r16;
-        const float sc = amax > 0.f ? amax / 448.f : 1.f;
-        const float inv = amax > 0.f ? 448.f / amax : 1.f;
-        const float inv16 = inv * 16.f;
+    for (int p = 0; p < 4; ++p) {
+        if (2 * p >= live) continue;
         uint32_t h[4], l[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const float* x = c[s][j];
-            h[j] = e4m3x4_from_f32(clamp448(x[0] * inv), clamp448(x[1] * inv),
-                                   clamp448(x[2] * inv), clamp448(x[3] * inv));
-            const auto h01 = __builtin_amdgcn_cvt_pk_f32_fp8((int)h[j], false);
-            const auto h23 = __builtin_amdgcn_cvt_pk_f32_fp8((int)h[j], true);
-            const float hv[4] = {h01[0], h01[1], h23[0], h23[1]};
-            float lq[4];
+        for (int q = 0; q < 2; ++q) {
+            const int s = 2 * p + q;
+            const int r = 128 * wm + 16 * s + r16;
+            float amax = 0.f;
 #pragma unroll
-            for (int v = 0; v < 4; ++v) lq[v] = clamp448(__builtin_fmaf(-hv[v], sc, x[v]) * inv16);
-            l[j] = e4m3x4_from_f32(lq[0], lq[1], lq[2], lq[3]);
+            for (int w = 0; w < 4; ++w) amax = fmaxf(amax, xch[w * 256 + r]);
+            const float sc = amax > 0.f ? amax / 448.f : 1.f;
+            const float inv = amax > 0.f ? 448.f / amax : 1.f;
+            const float inv16 = inv * 16.f;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const float* x = c[s][i];
+                const uint32_t hw = e4m3x4_from_f32(clamp448(x[0] * inv), clamp448(x[1] * inv),
+                                                    clamp448(x[2] * inv), clamp448(x[3] * inv));
+                const auto h01 = __builtin_amdgcn_cvt_pk_f32_fp8((int)hw, false);
+                const auto h23 = __builtin_amdgcn_cvt_pk_f32_fp8((int)hw, true);
+                const float hv[4] = {h01[0], h01[1], h23[0], h23[1]};
+                float lq[4];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) lq[v] = clamp448(__builtin_fmaf(-hv[v], sc, x[v]) * inv16);
+                h[2 * q + i] = hw;
+                l[2 * q + i] = e4m3x4_from_f32(lq[0], lq[1], lq[2], lq[3]);
+            }
+            if (wn == 0 && kq == 0 && r < nrows) C.scales[(size_t)ng * C.rows_cap + row0 + r] = sc;
         }
-        // every lane of the wave takes part in the swaps (the 4 lanes of a row share its
-        // validity); lane kq then holds bytes 16 kq .. 16 kq + 15 of the wave's 64
+        // every lane of the wave takes part in the swaps; lane kq then holds row block
+        // 2 p + kq / 2, columns 16 (kq & 1) .. + 15 of the wave's 32
         transpose4(h);
         transpose4(l);
+        const int r = 128 * wm + 16 * (2 * p + (kq >> 1)) + r16;
         if (r >= nrows) continue;
-        const size_t off = (size_t)(row0 + r) * kI + ng * 128 + 64 * wn + 16 * kq;
+        const size_t off = (size_t)(row0 + r) * kI + ng * 128 + 32 * wn + 16 * (kq & 1);
         *reinterpret_cast<v4u*>(C.hi() + off) = v4u{h[0], h[1], h[2], h[3]};
         *reinterpret_cast<v4u*>(C.lo() + off) = v4u{l[0], l[1], l[2], l[3]};
-        if (wn == 0 && kq == 0) C.scales[(size_t)ng * C.rows_cap + row0 + r] = sc;
     }
 }
 
 // ---------------------------------------------------------------------------
-// Prefill GEMM1 (many tokens per expert), MFMA-bound tiling: workgroup tile 256
-// gathered token rows x 256 weight rows (128 gate rows n0..n0+127 and the matching
-// 128 up rows 2048+n0.., i.e. 256 x 128 SwiGLU outputs), waves 4 (tokens) x 2
-// (weights), each 64 tokens x (64 gate + 64 up) rows: per K block 32 MFMA 16x16x128
-// (4 token blocks x 8 weight blocks) whose fresh partials are scaled by
-// sa[token] * sb[block] into fp32 accumulators.  Two waves per SIMD let one wave's
-// scale FMAs and LDS reads run under the other's MFMAs; registers stay <= 256 per
-// lane for that.  Two 66 KB stages; rows keep 16-byte chunk c at c ^ swz128(r), so
-// ds_read_b128 in the MFMA layout is conflict-free.  Padding row blocks skip their
-// MFMAs.  Items (row tile, 128-column group) follow prefill_items_ranked when `ranked`
-// is set, else grouped_item, with an XCD-contiguous mapping of each round.
+// Prefill GEMM1 (from a few dozen tokens per expert up): workgroup tile of up to 256
+// gathered token rows x 256 weight rows (128 gate rows n0 .. n0 + 127 and the matching 128
+// up rows 2048 + n0 .., i.e. 128 SwiGLU columns); waves 2 (token rows) x 4 (weight rows),
+// each 128 tokens x (32 gate + 32 up) rows: per K block up to 32 MFMA 16x16x128 (a wave
+// holds its 4 weight fragments and streams the token fragments past them) whose fresh
+// partials are scaled by sa[token] * sb[block] into fp32 accumulators.  Two waves per SIMD,
+// so registers stay <= 256 per lane.  Rows in LDS keep 16-byte chunk c at c ^ swz128(r), so
+// ds_read_b128 in the MFMA layout is conflict-free.  Items (row tile, 128-column group)
+// follow prefill_items_ranked, or grouped_item when that is not asked for or does not fit,
+// with an XCD-contiguous mapping of each round.
 //
-// Operand DMA is buffer_load ... lds (addresses in SGPR resources, 32-bit lane
-// offsets, the K step in the scalar offset), issued in two bursts per K block:
-// the token rows right after the barrier, the weight rows and token scales after
-// the third weight block's MFMAs, so the texture path is not flooded at once.
-// Each weight operand is read from LDS one block ahead of its MFMAs, and each fresh
-// partial is scaled into its accumulator only after the next weight block's MFMA of
-// the same token block has issued (fixed order), so no FMA waits on its MFMA.
-// A workgroup resolves the metadata of all its items at kernel start
-// (prefill_items) and issues the first stage of its next item at the top of the
-// current item's last K block; the epilogue's row-maximum exchange therefore uses
-// stage 1, which the last K block reads.
+// What bounds it.  An item of few rows is bound by its weight stream (32 KB per K block and
+// CU), one of many by the matrix cores at a clock the power limit holds to 1.9 GHz; both
+// lost their time waiting for operands: with two stages whatever the rows, a K block's loads
+// went out after the barrier that ended the block before and had to land by its own end.
+//   - The item's rows decide how many K blocks the LDS holds (Gemm1Class): the fewer rows,
+//     the deeper the weight stream runs ahead.
+//   - The barrier of a K block stands before its last token fragment's MFMAs, not after
+//     them: every fragment has been read by then, so the next block's first fragments are
+//     read under those MFMAs.
+//   - With two stages the weight stage is handed over earlier still, by a barrier of its own
+//     once every wave holds its weight fragments, so weight loads run 1.75 blocks ahead; the
+//     loads are spread over the block's MFMAs, as a wave that issues many back to back stalls
+//     on the address path (all at once: 3555 instead of 3345 cycles a K block with every
+//     operand in L2).
+//   - Past the last K block the buffers have no bytes: the loads stay in the loop without a
+//     branch, move nothing, and the counted waits hold in the last blocks too.
+// Measured (GEMM1, before -> after): 24 experts of 16 rows 173 -> 146 us, of 128 rows 205 ->
+// 182, of 256 rows 241 -> 226, of 512 rows 329 -> 323; uneven routings of T = 2731 259 ->
+// 214, T = 8192 385 -> 366 (335 ranked), skewed T = 4096 577 -> 550.
+// Not faster: 4 x 2 waves holding the token fragments (24 x 256 rows 236 us), 8 waves each
+// with its own 32 weight rows loaded straight into registers (half-line loads: 289 us).
+//
+// A workgroup resolves the metadata of all its items at kernel start; an item's token ids
+// and weight scales come by DMA during the item before, and its first K blocks are issued
+// before the epilogue of that item and land under it.
 // Token offsets are 32-bit: T * 7168 < 2^32 (T <= 2^19, checked by the host).
 // ---------------------------------------------------------------------------
+// Row class of an item, from its rows: how many K blocks of operands the LDS holds.
+//   A  145 .. 256 rows  2 stages of 32 KB token rows + 32 KB weight rows
+//   B   41 .. 144 rows  3 stages of 18 KB + 32 KB
+//   C    1 ..  40 rows  4 stages of  5 KB + 32 KB
+// (the rows at which the next deeper ring just fits into 160 KB beside the epilogue's and
+// the items' 9 KB)
+template <int NS, int ROWS, int NT>
+struct Gemm1Class {
+    static constexpr int kNS = NS;                     // stages
+    static constexpr int kNT = NT;                     // token-row loads per wave and K block
+    static constexpr int kRows = ROWS;
+    static constexpr int kSlots = (ROWS + 63) / 64 + 1;   // 64-row slots of token scales, and one for zeros
+    static constexpr int kTok = ROWS * kBlk;
+    static constexpr int kW = 256 * kBlk;
+    static constexpr int kTokBase = NS * kW;           // weight stages first
+    static constexpr int kScaBase = kTokBase + NS * kTok;
+    static constexpr int kBytes = kScaBase + NS * kSlots * 256;
+};
+// mode bits of gemm1_prefill8_kernel
+constexpr int kPrefillRanked = 1, kPrefillThroughF16 = 2;
+
+using Gemm1A = Gemm1Class<2, 256, 4>;
+using Gemm1B = Gemm1Class<3, 144, 3>;
+using Gemm1C = Gemm1Class<4, 40, 1>;
+
 struct Gemm1Item {   // uniform part of an item; the per-lane DMA offsets live apart
-    __amdgpu_buffer_rsrc_t w;
-    int le, row0, nrows, ng;
-    bool tok_live, sca_live;
+    const uint8_t* w;    // the expert's W1 from the item's first gate row on
+    uint32_t wbytes;
+    int row0, nrows, ng;
 };
 
 __global__ __launch_bounds__(512, 1) void gemm1_prefill8_kernel(
     const uint8_t* __restrict__ hidden, TokenScales sa, int T,
     const uint8_t* __restrict__ w1, const float* __restrict__ s1,
     const int4* __restrict__ tiles, const int* __restrict__ num_tiles,
-    const int* __restrict__ exp_off, const int* __restrict__ sorted_tok, Intermediate C, int ranked) {
-    constexpr int NS = 2;
+    const int* __restrict__ exp_off, const int* __restrict__ sorted_tok, Intermediate C, int mode) {
     constexpr int BM = 256;
     constexpr int NG = kI / 128;
-    constexpr int kA = BM * kBlk;               // 32 KB token rows
-    constexpr int kW = 256 * kBlk;              // 32 KB weight rows
-    constexpr int kStage = kA + kW + 8 * 256;   // + per-wave token-scale rows
-    constexpr int kWeightBurstAfter = 2;        // weight block after which burst 2 goes
-    constexpr int kItemCap = 1024;              // per-workgroup item table (16 KB of LDS)
-    static_assert(kHB % 2 == 0, "the next item's first stage must be stage 0");
-    // one LDS object: the stages, then the item table
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[NS * kStage + kItemCap * sizeof(int4)];
-    int4* const s_items = reinterpret_cast<int4*>(lds + NS * kStage);
+    constexpr int kItemCap = 64;                // per-workgroup item table
+    constexpr int kPool = std::max({Gemm1A::kBytes, Gemm1B::kBytes, Gemm1C::kBytes});
+    constexpr int kXch = kPool, kTokIds = kXch + 4 * BM * 4, kWsc = kTokIds + BM * 4, kItems = kWsc + 2 * 512;
+    // one LDS object: the stages, the row-maximum exchange, the next item's tokens, two
+    // items' weight scales, the item table
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[kItems + kItemCap * sizeof(int4)];
+    static_assert(sizeof(lds) <= 160 * 1024, "LDS of a CU");
+    int4* const s_items = reinterpret_cast<int4*>(lds + kItems);
+    const int* const s_tok = reinterpret_cast<const int*>(lds + kTokIds);
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const int r16 = lane & 15, kq = lane >> 4;
-    const int wm = wave >> 1, wn = wave & 1;
+    const int wm = wave >> 2, wn = wave & 3;
     const v4f zero = {0.f, 0.f, 0.f, 0.f};
     const int nitems = *num_tiles * NG;
     const int G = gridDim.x;
     const int base = (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3);   // XCD-contiguous slot
     const int drow = lane >> 3, dchunk = lane & 7;
     const int swz = swz128(r16);
-    const int c0 = ((2 * kq) ^ swz) << 4, c1 = ((2 * kq + 1) ^ swz) << 4;
-    const __amdgpu_buffer_rsrc_t rs_tok = buffer_rsrc(hidden, (uint32_t)T * kH);
-    const __amdgpu_buffer_rsrc_t rs_sca = buffer_rsrc(sa.p, (uint32_t)sa.stride * kHB * 4);
-    // wave w moves token rows 32w..32w+31 and weight rows 32w..32w+31 of the stage; the
-    // weight rows' lane offsets are relative to the item's first gate row (the resource
-    // base), so they do not depend on the item
+    const int c0 = r16 * kBlk + (((2 * kq) ^ swz) << 4), c1 = r16 * kBlk + (((2 * kq + 1) ^ swz) << 4);
+    const __amdgpu_buffer_rsrc_t rs_ids = buffer_rsrc(sorted_tok, (uint32_t)T * kTopK * 4);
+    const __amdgpu_buffer_rsrc_t rs_s1 = buffer_rsrc(s1, kEL * kN1B * kHB * 4);
+    constexpr uint32_t kNothing = 0xfffffff0u;   // an offset past every buffer: moves nothing
+    // wave w moves weight rows 32w..32w+31 of a stage; their lane offsets are relative to
+    // the item's first gate row (the resource base), so they do not depend on the item
     uint32_t woff[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -586,144 +632,267 @@ __global__ __launch_bounds__(512, 1) void gemm1_prefill8_kernel(
         woff[i] = (uint32_t)n * kH + ((dchunk ^ swz128(r)) << 4);
     }
 
-    static_assert(kRankThreads == 512 && kRankScratch <= NS * kStage, "ranked order: threads, scratch");
-    int nr = ranked ? prefill_items_ranked<BM>(s_items, kItemCap, NG, base, G, exp_off, lds) : -1;
+    static_assert(kRankThreads == 512 && kRankScratch <= kPool, "ranked order: threads, scratch");
+    int nr = (mode & kPrefillRanked) ? prefill_items_ranked<BM>(s_items, kItemCap, NG, base, G, exp_off, lds) : -1;
     if (nr < 0) nr = prefill_items<BM>(s_items, kItemCap, nitems, NG, base, G, tiles, exp_off);
     if (nr == 0) return;   // uniform: the whole workgroup has no item
     __syncthreads();
 
-    // token-row and token-scale offsets of the item whose stages are being fetched
-    uint32_t aoff[4], soff;
+    // lane-dependent addresses that only the change of items needs are computed there, from a
+    // lane number the compiler cannot see through: kept through the K loop they would spill,
+    // and a reload waits for every DMA in flight
+    auto opaque = [](int x) {
+        __asm__ volatile("" : "+v"(x));
+        return x;
+    };
+    // an item's tokens (waves 0..3, 64 each) and weight block scales (wave 4 gate, 5 up), by
+    // DMA into LDS; the scales of item r in buffer r & 1
+    auto fetch_side = [&](int r) {
+        const int4 m = prefill_item<BM>(s_items, kItemCap, r, NG, base, G, tiles, exp_off);
+        const int ln = opaque(lane);
+        if (wave < 4) {
+            bdma4(rs_ids, (uint32_t)(m.y + min(64 * wave + ln, m.z - 1)) * 4, 0, lds + kTokIds + wave * 256);
+        } else if (wave < 6) {
+            const uint32_t first = (uint32_t)(m.x * kN1B + m.w + (wave == 5 ? kIB : 0)) * kHB;
+            bdma4(rs_s1, (first + min(ln, kHB - 1)) * 4, 0, lds + kWsc + (r & 1) * 512 + (wave - 4) * 256);
+        }
+    };
+    uint32_t aoff[4], soff;   // token-row and token-scale offsets of the item being fetched
     auto make_item = [&](int r) {
         const int4 m = prefill_item<BM>(s_items, kItemCap, r, NG, base, G, tiles, exp_off);
         Gemm1Item it;
-        it.le = m.x;
         it.row0 = m.y;
         it.nrows = m.z;
         it.ng = m.w;
-        const size_t first = (size_t)it.le * kN1 + (size_t)it.ng * 128;
-        it.w = buffer_rsrc(w1 + first * kH, (uint32_t)(((size_t)(it.le + 1) * kN1 - first) * kH));
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int r = 32 * wave + 8 * i + drow;
-            const int tok = sorted_tok[it.row0 + min(r, it.nrows - 1)];
-            aoff[i] = (uint32_t)tok * kH + ((dchunk ^ swz128(r)) << 4);
-        }
-        const int srow = it.row0 + min(64 * wm + lane, it.nrows - 1);
-        soff = (uint32_t)(sa.by_row ? srow : sorted_tok[srow]) * 4;
-        // a wave whose 32 token rows all lie past the tile moves nothing: they would only
-        // repeat the last row, and the MFMAs of their 16-row blocks are skipped
-        it.tok_live = 32 * wave < it.nrows;
-        it.sca_live = 64 * wm < it.nrows;
+        const size_t first = (size_t)m.x * kN1 + (size_t)it.ng * 128;
+        it.w = w1 + first * kH;
+        it.wbytes = (uint32_t)(((size_t)(m.x + 1) * kN1 - first) * kH);
         return it;
     };
-    auto issue_tokens = [&](const Gemm1Item& it, int kb) {
-        uint8_t* st = lds + (kb & 1) * kStage;
-        if (it.tok_live) {
+    // 8-row blocks of token rows this wave moves: NT wave + i (clamped into the class's rows,
+    // the clamped ones moving the last block again)
+    auto tok_block = [&](auto cls, int i) {
+        using Cl = decltype(cls);
+        return min(Cl::kNT * wave + i, Cl::kRows / 8 - 1);
+    };
+    auto set_offsets = [&](auto cls, const Gemm1Item& it) {
+        using Cl = decltype(cls);
+        const int ln = opaque(lane);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) bdma16(rs_tok, aoff[i], (uint32_t)kb * kBlk, st + (32 * wave + 8 * i) * kBlk);
+        for (int i = 0; i < Cl::kNT; ++i) {
+            const int q = tok_block(cls, i);
+            const int r = 8 * q + (ln >> 3);
+            // a block past the tile moves nothing
+            aoff[i] = 8 * q < it.nrows ? (uint32_t)s_tok[min(r, it.nrows - 1)] * kH + (((ln & 7) ^ swz128(r)) << 4)
+                                       : kNothing;
+        }
+        const int sr = min(64 * wave + ln, it.nrows - 1);
+        soff = 64 * wave < it.nrows ? (uint32_t)(sa.by_row ? it.row0 + sr : s_tok[sr & 255]) * 4 : kNothing;
+    };
+    // K block kb of an item into a stage; past the last block the buffers have no bytes, so
+    // that nothing moves and the number of loads in flight stays the same without a branch
+    // in the K loop
+    auto issue_w = [&](auto cls, const Gemm1Item& it, int kb, int stage, int i0 = 0, int i1 = 4) {
+        using Cl = decltype(cls);
+        const __amdgpu_buffer_rsrc_t rs_w = buffer_rsrc(it.w, kb < kHB ? it.wbytes : 0u);
+#pragma unroll
+        for (int i = i0; i < i1; ++i)
+            bdma16(rs_w, woff[i], (uint32_t)kb * kBlk, lds + stage * Cl::kW + (32 * wave + 8 * i) * kBlk);
+    };
+    auto issue_t = [&](auto cls, int kb, int stage, int i0 = 0, int i1 = 5) {
+        using Cl = decltype(cls);
+        const bool on = kb < kHB;
+        const __amdgpu_buffer_rsrc_t rs_tok = buffer_rsrc(hidden, on ? (uint32_t)T * kH : 0u);
+        const __amdgpu_buffer_rsrc_t rs_sca = buffer_rsrc(sa.p, on ? (uint32_t)sa.stride * kHB * 4 : 0u);
+#pragma unroll
+        for (int i = i0; i < i1 && i < Cl::kNT; ++i)
+            bdma16(rs_tok, aoff[i], (uint32_t)kb * kBlk, lds + Cl::kTokBase + stage * Cl::kTok + 8 * tok_block(cls, i) * kBlk);
+        if (i1 == 5)
+        bdma4(rs_sca, soff, (uint32_t)kb * sa.stride * 4,
+              lds + Cl::kScaBase + (stage * Cl::kSlots + min(wave, Cl::kSlots - 1)) * 256);
+    };
+    auto start = [&](auto cls, const Gemm1Item& it) {   // the item's first stages
+        set_offsets(cls, it);
+#pragma unroll
+        for (int k = 0; k < decltype(cls)::kNS; ++k) {
+            issue_w(cls, it, k, k);
+            if (decltype(cls)::kNS > 2 || k == 0) issue_t(cls, k, k);
+            else issue_t(cls, k, k, 0, 2);   // the rest in the K loop
         }
     };
-    auto issue_weights = [&](const Gemm1Item& it, int kb) {
-        uint8_t* st = lds + (kb & 1) * kStage;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) bdma16(it.w, woff[i], (uint32_t)kb * kBlk, st + kA + (32 * wave + 8 * i) * kBlk);
-        if (it.sca_live) bdma4(rs_sca, soff, (uint32_t)kb * sa.stride * 4, st + kA + kW + wave * 256);
+    auto with_class = [&](int nrows, auto&& f) {
+        if (nrows > Gemm1B::kRows) f(Gemm1A{});
+        else if (nrows > Gemm1C::kRows) f(Gemm1B{});
+        else f(Gemm1C{});
     };
 
+    fetch_side(0);
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+    lds_barrier();
     Gemm1Item cur = make_item(0), nxt = cur;
-    issue_tokens(cur, 0);
-    issue_weights(cur, 0);
+    with_class(cur.nrows, [&](auto cls) { start(cls, cur); });
     for (int r = 0; r < nr; ++r) {
         const bool more = r + 1 < nr;
-        // weight block scales of the gate and up rows (scalar loads from the kernel argument)
-        const float* sgp = s1 + (size_t)(cur.le * kN1B + cur.ng) * kHB;
-        const float* sup = sgp + (size_t)kIB * kHB;
-        v4f acc[4][8];
+        const float* const wsc = reinterpret_cast<const float*>(lds + kWsc + (r & 1) * 512);
+        v4f acc[8][4];
 #pragma unroll
-        for (int s = 0; s < 4; ++s)
+        for (int s = 0; s < 8; ++s)
 #pragma unroll
-            for (int j = 0; j < 8; ++j) acc[s][j] = zero;
+            for (int i = 0; i < 4; ++i) acc[s][i] = zero;
 
-        // token rows 64 wm + 16 s .. of this wave that exist: the MFMAs of padding
-        // blocks are skipped (the DMA and barriers stay the same for every wave)
-        auto kloop = [&](auto live) {
-        constexpr int NLIVE = decltype(live)::value;
-        constexpr int NT = NLIVE > 0 ? NLIVE : 1;
-#pragma unroll 1
-        for (int kb = 0; kb < kHB; ++kb) {
-            __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-            __syncthreads();
-            if (kb + 1 < kHB) {
-                issue_tokens(cur, kb + 1);
-                if (kWeightBurstAfter < 0 || NLIVE == 0) issue_weights(cur, kb + 1);
-            } else if (more) {
-                // stage 0 is free (every wave is past K block kHB - 2): the next item's first stage
-                nxt = make_item(r + 1);
-                issue_tokens(nxt, 0);
-                issue_weights(nxt, 0);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            if (NLIVE == 0) continue;
-
-            const uint8_t* st = lds + (kb & 1) * kStage;
-            const float fsg = sgp[kb], fsu = sup[kb];
-            const float* sar = reinterpret_cast<const float*>(st + kA + kW + wave * 256);
-            v8i bt[4];
-            float fg[4], fu[4];
-#pragma unroll
-            for (int s = 0; s < NLIVE; ++s) {
-                const uint8_t* rp = st + (64 * wm + 16 * s + r16) * kBlk;
-                const v4u x0 = *reinterpret_cast<const v4u*>(rp + c0);
-                const v4u x1 = *reinterpret_cast<const v4u*>(rp + c1);
-                bt[s] = v8i{(int)x0[0], (int)x0[1], (int)x0[2], (int)x0[3], (int)x1[0], (int)x1[1], (int)x1[2], (int)x1[3]};
-                const float sa = sar[16 * s + r16];
-                fg[s] = sa * fsg;
-                fu[s] = sa * fsu;
-            }
-            auto read_w = [&](int j) {
-                const int r = (j < 4) ? (64 * wn + 16 * j) : (128 + 64 * wn + 16 * (j - 4));
-                const uint8_t* rp = st + kA + (r + r16) * kBlk;
+        // NL: row blocks 128 wm + 16 j of this wave that are computed (the live ones, rounded
+        // up to the instantiated counts; padding rows are computed on whatever the LDS holds
+        // and never stored)
+        auto kloop = [&](auto cls, auto live) {
+            using Cl = decltype(cls);
+            constexpr int NL = decltype(live)::value;
+            constexpr int NS = Cl::kNS;
+            auto rd = [&](const uint8_t* rp) {
                 const v4u x0 = *reinterpret_cast<const v4u*>(rp + c0);
                 const v4u x1 = *reinterpret_cast<const v4u*>(rp + c1);
                 return v8i{(int)x0[0], (int)x0[1], (int)x0[2], (int)x0[3], (int)x1[0], (int)x1[1], (int)x1[2], (int)x1[3]};
             };
-            v8i bw = read_w(0);
-            v4f tp[NT];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                v8i bwn = bw;
-                if (j < 7) bwn = read_w(j + 1);
-                if (j == kWeightBurstAfter && kb + 1 < kHB) {
-                    __builtin_amdgcn_sched_barrier(0);
-                    issue_weights(cur, kb + 1);
-                }
-#pragma unroll
-                for (int s = 0; s < NLIVE; ++s) {
-                    __builtin_amdgcn_sched_barrier(0);
-                    const v4f tc = mfma_fp8(bw, bt[s], zero);
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (j > 0) {
-                        const float f = (j - 1 < 4) ? fg[s] : fu[s];
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) acc[s][j - 1][v] = __builtin_fmaf(tp[s][v], f, acc[s][j - 1][v]);
+            auto read_t = [&](int stage, int j) {
+                return rd(lds + Cl::kTokBase + stage * Cl::kTok + (128 * wm + 16 * j) * kBlk);
+            };
+            auto read_s = [&](int stage, int j) {
+                return reinterpret_cast<const float*>(lds + Cl::kScaBase + stage * Cl::kSlots * 256)[128 * wm + 16 * j + r16];
+            };
+            auto read_w = [&](int stage, int i) {
+                return rd(lds + stage * Cl::kW + ((i < 2 ? 0 : 128) + 32 * wn + 16 * (i & 1)) * kBlk);
+            };
+            // kEarly (two stages): a K block's weight stage is handed over by a barrier of its
+            // own, as soon as every wave holds the block's weight fragments, and the loads are
+            // spread over the block's MFMAs.  Otherwise both stages go with the barrier before
+            // the last token block's MFMAs, all loads right after it.
+            constexpr bool kEarly = NS == 2;
+            constexpr int kFirstT = kEarly ? 2 : 5;   // token loads right after the hand-over
+            // every wave holds its weight fragments of K block kb: the weight stage goes to
+            // block kb + NS
+            auto free_weights = [&](int kb, int stage) {
+                __builtin_amdgcn_sched_barrier(0);
+                lds_barrier();
+                if (NL > 4) issue_w(cls, cur, kb + NS, stage, 0, 1);
+                else issue_w(cls, cur, kb + NS, stage);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            // every wave has read its last token fragment of K block kb, and block kb + 1 has
+            // landed for every wave: the token stage goes to block kb + NS
+            auto hand_over = [&](int kb, int stage) {
+                __builtin_amdgcn_sched_barrier(0);
+                __builtin_amdgcn_s_waitcnt(vmcnt_imm(kEarly ? 4 : (NS - 2) * (4 + Cl::kNT + 1)));
+                lds_barrier();
+                if (!kEarly) issue_w(cls, cur, kb + NS, stage);
+                issue_t(cls, kb + NS, stage, 0, kFirstT);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            if (kEarly) __builtin_amdgcn_s_waitcnt(vmcnt_imm(4 + 2));
+            else __builtin_amdgcn_s_waitcnt(vmcnt_imm((NS - 1) * (4 + Cl::kNT + 1)));
+            lds_barrier();
+            if (more) fetch_side(r + 1);
+            int stage = 0;
+            if constexpr (NL == 0) {
+#pragma unroll 1
+                for (int kb = 0; kb < kHB; ++kb) {
+                    if (kEarly) {
+                        issue_t(cls, kb - 1 + NS, stage == 0 ? NS - 1 : stage - 1, 2, 5);
+                        free_weights(kb, stage);
                     }
-                    tp[s] = tc;
+                    hand_over(kb, stage);
+                    stage = stage + 1 == NS ? 0 : stage + 1;
                 }
-                bw = bwn;
+            } else {
+                int first = 0;
+                __asm__ volatile("" : "+s"(first));   // as opaque()
+                v8i w[4];
+                v8i t = read_t(first, 0);
+                float sv = read_s(first, 0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) w[i] = read_w(first, i);
+                float wg = wsc[0], wu = wsc[64];
+                v4f tp[4];
+                float fgp = 0.f, fup = 0.f;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) tp[i] = zero;
+#pragma unroll 1
+                for (int kb = 0; kb < kHB; ++kb) {
+                    const int nstage = stage + 1 == NS ? 0 : stage + 1;
+                    const int pstage = stage == 0 ? NS - 1 : stage - 1;
+                    float wgn = 0.f, wun = 0.f;
+#pragma unroll
+                    for (int j = 0; j < NL; ++j) {
+                        if (kEarly && j == 1) free_weights(kb, stage);
+                        v8i tn;
+                        float svn;
+                        if (j < NL - 1) {
+                            tn = read_t(stage, j + 1);
+                            svn = read_s(stage, j + 1);
+                        } else {
+                            hand_over(kb, stage);
+                            tn = read_t(nstage, 0);
+                            svn = read_s(nstage, 0);
+                            wgn = wsc[kb + 1];
+                            wun = wsc[64 + kb + 1];
+                        }
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            __builtin_amdgcn_sched_barrier(0);
+                            const v4f tc = mfma_fp8(w[i], t, zero);
+                            __builtin_amdgcn_sched_barrier(0);
+                            if (j == NL - 1) w[i] = read_w(nstage, i);
+                            const int jp = (j + NL - 1) % NL;
+                            const float f = i < 2 ? fgp : fup;
+#pragma unroll
+                            for (int v = 0; v < 4; ++v) acc[jp][i][v] = __builtin_fmaf(tp[i][v], f, acc[jp][i][v]);
+                            tp[i] = tc;
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                        if (kEarly && j == 0) issue_t(cls, kb - 1 + NS, pstage, 2, 5);
+                        if (kEarly && NL > 4 && j >= 1 && j <= 3) issue_w(cls, cur, kb + NS, stage, j, j + 1);
+                        __builtin_amdgcn_sched_barrier(0);
+                        fgp = sv * wg;
+                        fup = sv * wu;
+                        t = tn;
+                        sv = svn;
+                    }
+                    wg = wgn;
+                    wu = wun;
+                    stage = nstage;
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        acc[NL - 1][i][v] = __builtin_fmaf(tp[i][v], i < 2 ? fgp : fup, acc[NL - 1][i][v]);
             }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int s = 0; s < NLIVE; ++s)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) acc[s][7][v] = __builtin_fmaf(tp[s][v], fu[s], acc[s][7][v]);
-        }
         };
-        with_live_blocks(live_blocks(64 * wm, cur.nrows), kloop);
+        const int live = min(8, max(0, (cur.nrows - 128 * wm + 15) >> 4));
+        if (cur.nrows > Gemm1B::kRows) {
+            if (live > 6) kloop(Gemm1A{}, IntC<8>{});
+            else if (live > 4) kloop(Gemm1A{}, IntC<6>{});
+            else if (live > 2) kloop(Gemm1A{}, IntC<4>{});
+            else kloop(Gemm1A{}, IntC<2>{});
+        } else if (cur.nrows > Gemm1C::kRows) {
+            if (live > 6) kloop(Gemm1B{}, IntC<8>{});
+            else if (live > 4) kloop(Gemm1B{}, IntC<6>{});
+            else if (live > 1) kloop(Gemm1B{}, IntC<4>{});
+            else if (live == 1) kloop(Gemm1B{}, IntC<1>{});
+            else kloop(Gemm1B{}, IntC<0>{});
+        } else {
+            if (live > 1) kloop(Gemm1C{}, IntC<3>{});
+            else if (live == 1) kloop(Gemm1C{}, IntC<1>{});
+            else kloop(Gemm1C{}, IntC<0>{});
+        }
 
-        // the next item's first stage is landing in stage 0: the exchange uses stage 1
-        store_c_hilo(acc, reinterpret_cast<float*>(lds + kStage), wm, wn, kq, r16, cur.row0, cur.nrows,
-                     cur.ng, C);
+        // every stage is free (each wave has passed the last block's barrier): the next
+        // item's first blocks land under this item's epilogue
+        if (more) {
+            nxt = make_item(r + 1);
+            with_class(nxt.nrows, [&](auto cls) { start(cls, nxt); });
+        }
+        store_c_hilo(acc, reinterpret_cast<float*>(lds + kXch), live, wm, wn, kq, r16, cur.row0, cur.nrows,
+                     cur.ng, C, mode & kPrefillThroughF16);
         cur = nxt;
     }
 }
@@ -800,7 +969,7 @@ bool launch_gemm1_dispatch(const RouteIn& rin, int* topk_ids, float* topk_w, int
 bool launch_gemm1(int variant, const uint8_t* hidden, const TokenScales& sa, int T,
                   const uint8_t* w1, const float* s1, const int4* tiles, const int* num_tiles,
                   const int* exp_off, int max_tiles, const int* sorted_tok, const Intermediate& C,
-                  bool ranked, hipStream_t stream) {
+                  bool ranked, bool through_f16, hipStream_t stream) {
     int* c_wide = const_cast<int*>(exp_off) + kCWideFlag;   // meta word, cleared by the route kernel
     const int prefill_grid = 256;   // one resident workgroup per CU (LDS-bound)
     constexpr int G = kI / 16;      // 16-column groups
@@ -829,7 +998,7 @@ bool launch_gemm1(int variant, const uint8_t* hidden, const TokenScales& sa, int
         case 4:
             launch_kernel(gemm1_prefill8_kernel, dim3(prefill_grid), dim3(512), 0, stream,
                                hidden, sa, T, w1, s1, tiles, num_tiles, exp_off, sorted_tok, C,
-                               ranked ? 1 : 0);
+                               (ranked ? kPrefillRanked : 0) | (through_f16 ? kPrefillThroughF16 : 0));
             return true;
         default: return false;
     }

@@ -35,12 +35,11 @@ constexpr int kMinTileM = 16;           // smallest row tile; sizes the tile lis
 // runs three or two workgroups per CU as the call's tile count makes best), feeding up to
 // T = 559 the token-sharing GEMM2 on the same tiles (variant 7: fp16 C, no conversion;
 // 1-13 us faster than the neighbouring pairs at T = 200 .. 560 over three routings) and
-// beyond the prefill GEMM2 (128-row tiles, FP8 MFMA on the hi/lo form); from T = 1345 both
+// beyond the prefill GEMM2 (128-row tiles, FP8 MFMA on the hi/lo form), from T = 700 with
+// the prefill GEMM1 in its place (row_class); from T = 1345 both
 // GEMMs are the MFMA-bound prefill kernels on 256-row tiles (GEMM2 on the 128-row second
 // list).  The boundaries come from wall-clock sweeps of the pairs at T = 72 .. 2560 on
-// MI355X over routing seeds from light to heavy routing to the local experts.  Between T = 961 and
-// 1344 variant 8 was 6-25 us faster than variant 7 (always two per CU) on three routings
-// and 4-10 us slower on three; heavier routing there can prefer the prefill pair.
+// MI355X over routing seeds from light to heavy routing to the local experts.
 struct Plan {
     int tm;        // tile height of the first list
     int tm2;       // tile height of the second list (0: none)
@@ -50,11 +49,23 @@ struct Plan {
     bool dispatch_in_gemm1;   // GEMM1 variant 5 computes the dispatch itself (no launch)
     bool combine_in_gemm2;    // GEMM2 variant 6 writes the output itself (no combine launch)
     bool route_in_gemm1;      // GEMM1 variant 9 routes the tokens itself (no route launch)
+    bool row_class;           // pair 8/5 with the prefill GEMM1 in variant 8's place
 };
 
 inline int g1_tile_m(int v) { return v == 1 || v == 5 || v == 9 ? 16 : v == 2 ? 32 : v == 7 || v == 8 ? 64 : 256; }
 inline bool g1_hilo(int v) { return v == 4; }        // GEMM1 writes the hi/lo form
 inline bool g2_hilo(int v) { return v == 5; }        // GEMM2 reads the hi/lo form (7: fp16)
+
+// Pair 8/5 runs the prefill GEMM1 in the place of the token-sharing one from T =
+// kRowClassMinT on: the same fp32 sums, rounded through fp16, written as the hi/lo form the
+// conversion would make of them (bit-identical rows, no conversion launch).  It orders its
+// items by the expert offsets alone, so the pair's 64-row tile list stays what it was.  Both
+// sides measured (GEMM1 + conversion + GEMM2 and the rest, four routings each, us): T = 560
+// 206-233 token-sharing, 216-239 prefill; 700 231-253, 227-245; 850 244-274, 232-254; 1000
+// 250-292, 238-262; 1344 287-349, 246-277.  The bound above keeps the ranked order's tables
+// (kRankMaxGroups groups, the kernel's 64 rounds) from running out.
+constexpr int32_t kRowClassMinT = 700;
+constexpr int32_t kRowClassMaxT = 16384;
 
 // The plan of a GEMM1 / GEMM2 pair, false when they cannot run together.  GEMM1
 // variant 5 is variant 1 with the dispatch folded in (T <= 64): every workgroup of a
@@ -89,7 +100,8 @@ inline bool make_plan(int g1, int g2, int32_t T, Plan* p) {
     const int tm = g1_tile_m(g1);
     if (g1_hilo(g1) && !g2_hilo(g2)) return false;      // the fp16 GEMM2s need fp16 C
     if (g2 == 5) {                                       // the second list, 128-row tiles
-        *p = {tm, 128, g1, g2, !g1_hilo(g1), false, false, false};
+        const bool rc = g1 == 8 && T >= kRowClassMinT && T <= kRowClassMaxT;
+        *p = {tm, 128, g1, g2, !g1_hilo(g1) && !rc, false, false, false, false, rc};
         return true;
     }
     const int tm_g2 = g2 == 1 ? 16 : 32;
@@ -104,12 +116,6 @@ inline bool make_plan(int g1, int g2, int32_t T, Plan* p) {
 // gathering DMA instruction either way, so it reads them by token and the gather launch
 // goes away (-1 us at T = 600 .. 1280).
 constexpr int32_t kRowScalesMinT = 512;
-
-// The prefill GEMM1 takes its items ranked by expert rows (prefill_items_ranked) up to
-// T = kRankedMaxT and in tile-list order beyond.  Measured on three routings each at
-// T = 1400 .. 3500 the ranked order was 4-24 us faster on 17 of 21 (GEMM1 ~180-270 us)
-// and at most 6 us slower; at T = 4096 (skewed), 5000 and 8192 it was 4-19 us slower.
-constexpr int32_t kRankedMaxT = 3500;
 
 // GEMM2 computes the combine itself (variant 6, after GEMM1 variant 5) up to T =
 // kFusedCombinePlanMaxT, though it can up to kFusedCombineMaxT: measured against GEMM2
@@ -146,7 +152,7 @@ inline int plan_for(int32_t T, int32_t flags, Plan* p) {
     }
     if (!make_plan(g1, g2, T, p)) return MOE_ERR_BAD_FLAGS;
     if (on && (off || p->dispatch_in_gemm1)) return MOE_ERR_BAD_FLAGS;
-    p->by_row = on ? true : off ? false : (T >= kRowScalesMinT && p->g1 != 7 && p->g1 != 8);
+    p->by_row = on ? true : off ? false : (T >= kRowScalesMinT && (p->row_class || (p->g1 != 7 && p->g1 != 8)));
     return MOE_OK;
 }
 
@@ -194,7 +200,7 @@ inline int fill_layout(int32_t T, int32_t flags, moe_mi355_workspace_layout* L) 
     if (st != MOE_OK) return st;
     *L = workspace_regions(T);
     L->tile_m = plan.tm;
-    L->intermediate_format = g1_hilo(plan.g1) ? 1 : plan.convert ? 2 : 0;
+    L->intermediate_format = g1_hilo(plan.g1) ? 1 : plan.convert || plan.row_class ? 2 : 0;
     L->dispatch_in_gemm1 = plan.dispatch_in_gemm1 ? 1 : 0;
     L->combine_in_gemm2 = plan.combine_in_gemm2 ? 1 : 0;
     return MOE_OK;

@@ -112,7 +112,9 @@ typedef struct moe_mi355_args {
  *                                  (pairs with GEMM2 5 and 7 only), two workgroups per
  *                                  CU, 8 the same held to three per CU, of which it runs
  *                                  three or two by the call's tile count (the default
- *                                  for 200 <= T <= 1344);
+ *                                  for 200 <= T <= 1344; in pair 8/5 from T = 700 on the
+ *                                  prefill kernel computes the same rows in its place,
+ *                                  bit-identical, and writes the hi/lo form itself);
  *                                  GEMM2: 1 streaming 16-row, 3 streaming 32-row,
  *                                  5 prefill on a second list of 128-row tiles (the
  *                                  default for 560 <= T), 7 streaming with shared C
@@ -141,9 +143,8 @@ typedef struct moe_mi355_args {
  *                                  separate dispatch at T <= 64 (and is an error with
  *                                  variant 5 or 9 forced).
  *   MOE_MI355_FLAG_LIST_ORDER      the prefill GEMM1 (variant 4) takes its work items in
- *                                  tile-list order also at T <= 3500 (by default it
- *                                  ranks them by expert rows there, which balances the
- *                                  workgroups' loads); which workgroup computes an item
+ *                                  tile-list order (by default it ranks them by expert
+ *                                  rows, which balances the workgroups' loads); which workgroup computes an item
  *                                  is all that changes, so the output is bit-identical
  *                                  either way.
  * Every variant meets the same tolerance; the flags change speed only. */
@@ -263,7 +264,9 @@ typedef struct moe_mi355_workspace_layout {
                                   fp16(C 2^-e); e = 0 unless the group holds a value
                                   beyond the fp16 range (meta[35] set).
                                intermediate_format: 0 fp16 form, 1 hi/lo form, 2 fp16
-                               form converted to the hi/lo form before GEMM2 */
+                               form converted to the hi/lo form before GEMM2 (pair
+                               8/5 from T = 700 on writes those hi/lo rows directly,
+                               and no fp16 form) */
     size_t intermediate_scales; /* fp32 [16, 8T]: s of row r, 128-column block b at [b][r] */
     size_t expert_out;      /* fp16  [8T, 7168]  GEMM2 output rows */
     size_t expert_out_exp;  /* uint8 [8T, 448]   their 16-column group exponents, as for

@@ -1,0 +1,92 @@
+"""The prefill GEMM1's row classes (how deep its operand rings run by the rows of an item)
+at their edges: experts with exactly the row counts where a 16-row block, a class (40 / 41,
+144 / 145) or a 256-row tile begins or ends, checked row by row against the fp32 oracle, and
+pair 8/5 from T = 700 on, where this kernel stands in for the token-sharing GEMM1, against
+pair 7/5, whose C goes through fp16 and the conversion: bit-identical outputs."""
+import pytest
+import torch
+
+from conftest import oracle, pkg
+from gpu_common import config_inputs, note
+
+pytestmark = pytest.mark.gpu
+
+EDGES = (1, 15, 16, 17, 32, 33, 39, 40, 41, 47, 48, 49, 64, 65, 127, 128, 129, 143, 144, 145,
+         0, 160, 161, 239, 240, 241, 255, 256, 257, 0, 296, 397)
+SMALL = (1, 16, 17, 0, 40, 41, 64, 65, 128, 0, 129, 144, 145, 0, 64)   # 854 tokens
+
+
+def _inputs(counts):
+    """One local expert per token, counts[e] tokens for local expert e in a shuffled order;
+    the other seven picks are experts of groups 1 .. 3 (not local at offset 0)."""
+    wl = pkg("workloads")
+    T = sum(counts)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(40 + T)
+    lg = -6.0 + 0.01 * torch.randn(T, 256, generator=g, device="cuda")
+    e = torch.repeat_interleave(torch.arange(len(counts), device="cuda"),
+                                torch.tensor(counts, device="cuda"))
+    e = e[torch.randperm(T, generator=g, device="cuda")]
+    lg[torch.arange(T, device="cuda"), e] = 3.0
+    for j in range(7):
+        lg[:, 32 * (1 + j % 3) + 5 * j] = 2.0 + 0.1 * j
+    hs, sc = wl.quantize_rows_128(torch.randn(T, 7168, generator=g, device="cuda").to(torch.bfloat16))
+    d = dict(config_inputs(3))
+    d.update(routing_logits=lg, routing_bias=torch.zeros(256, dtype=torch.bfloat16, device="cuda"),
+             hidden_states=hs, hidden_states_scale=sc, local_expert_offset=0,
+             output=torch.empty(T, 7168, dtype=torch.bfloat16, device="cuda"))
+    return d, T
+
+
+def _run(d, T, flags):
+    k = pkg("kernel")
+    wl = pkg("workloads")
+    lay = k.workspace_layout(T, flags)
+    ws = torch.full((lay.total,), 255, dtype=torch.uint8, device="cuda")   # fp8 / fp16 NaN
+    out = torch.full_like(d["output"], float("nan"))
+    k.forward(*wl.as_args({**d, "output": out}), workspace=ws, flags=flags)
+    torch.cuda.synchronize()
+    assert not torch.isnan(out).any()
+    return lay, ws, out
+
+
+@pytest.mark.parametrize("scales", ["gathered", "by token"])
+def test_row_counts_at_the_class_edges(scales):
+    k = pkg("kernel")
+    o = oracle()
+    d, T = _inputs(EDGES)
+    note(f"[gpu] row classes T={T} scales {scales}")
+    lay, ws, _ = _run(d, T, k.FLAG_ROW_SCALES_OFF if scales == "by token" else 0)
+    assert lay.tile_m == 256
+    R = T * 8
+    off = ws[lay.meta:lay.meta + 33 * 4].view(torch.int32).cpu().tolist()
+    assert [off[e + 1] - off[e] for e in range(32)] == list(EDGES)
+    stok = ws[lay.sorted_tokens:lay.sorted_tokens + off[32] * 4].view(torch.int32).cpu().tolist()
+    hi = ws[lay.intermediate:lay.intermediate + R * 2048].view(R, 2048)
+    lo = ws[lay.intermediate + R * 2048:lay.intermediate + 2 * R * 2048].view(R, 2048)
+    sc = ws[lay.intermediate_scales:lay.intermediate_scales + 16 * R * 4].view(torch.float32).view(16, R)
+    for e, n in enumerate(EDGES):
+        # first, last and block- or tile-edge rows of the expert
+        rows = sorted({off[e] + r for r in (0, 15, 16, 127, 128, 255, 256, n // 2, n - 1) if 0 <= r < n})
+        if not rows:
+            continue
+        idx = torch.tensor(rows, device="cuda")
+        got = o.hilo_join(hi[idx].cpu(), lo[idx].cpu(), sc[:, idx].t().contiguous().cpu())
+        ref = o.swiglu_rows(d["hidden_states"], d["hidden_states_scale"], d["gemm1_weights"],
+                            d["gemm1_weights_scale"], e, [stok[r] for r in rows])
+        # hi + lo/16 of e4m3 parts holds a value to 2^-8 of itself or of its block's maximum
+        # (lo's own granule); twice that, for the fp32 sums' order
+        bmax = ref.view(-1, 16, 128).abs().amax(dim=2).repeat_interleave(128, dim=1)
+        err = (got - ref).abs()
+        assert (err <= ref.abs() * 2.0 ** -7 + bmax * 2.0 ** -10).all(), (e, n, float(err.max()))
+
+
+def test_pair_8_5_is_bit_identical_to_7_5():
+    k = pkg("kernel")
+    d, T = _inputs(SMALL)
+    assert T >= 700
+    note(f"[gpu] pair 8/5 by row classes T={T}")
+    _, _, ref = _run(d, T, k.plan_flags(7, 5))
+    for flags in (0, k.plan_flags(8, 5), k.FLAG_LIST_ORDER, k.FLAG_ROW_SCALES_OFF, k.FLAG_ROW_SCALES_ON):
+        _, _, out = _run(d, T, flags)
+        assert torch.equal(out.view(torch.int16), ref.view(torch.int16)), flags
