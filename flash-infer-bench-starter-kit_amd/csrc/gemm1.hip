@@ -886,8 +886,12 @@ __global__ __launch_bounds__(512, 1) void gemm1_prefill8_kernel(
         }
 
         // every stage is free (each wave has passed the last block's barrier): the next
-        // item's first blocks land under this item's epilogue
+        // item's first blocks land under this item's epilogue.  The loads past the last block,
+        // which still write zeros into the stages, are waited for first: the stages of an item
+        // of another class overlap those of other waves.
         if (more) {
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+            lds_barrier();
             nxt = make_item(r + 1);
             with_class(nxt.nrows, [&](auto cls) { start(cls, nxt); });
         }
