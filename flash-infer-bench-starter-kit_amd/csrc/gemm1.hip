@@ -547,11 +547,16 @@ __device__ __forceinline__ void store_c_hilo(const v4f (&acc)[8][4], float* xch,
 //     loads are spread over the block's MFMAs, as a wave that issues many back to back stalls
 //     on the address path (all at once: 3555 instead of 3345 cycles a K block with every
 //     operand in L2).
+//   - Weights that only this item's workgroup reads (the expert has one row tile) are loaded
+//     non-temporal up to T = kOnceMaxT; those of an expert with more tiles are not, its tiles
+//     meet in L2.
 //   - Past the last K block the buffers have no bytes: the loads stay in the loop without a
 //     branch, move nothing, and the counted waits hold in the last blocks too.
 // Measured (GEMM1, before -> after): 24 experts of 16 rows 173 -> 146 us, of 128 rows 205 ->
 // 182, of 256 rows 241 -> 226, of 512 rows 329 -> 323; uneven routings of T = 2731 259 ->
-// 214, T = 8192 385 -> 366 (335 ranked), skewed T = 4096 577 -> 550.
+// 214, T = 8192 385 -> 366 (335 ranked), skewed T = 4096 577 -> 550.  The non-temporal loads
+// alone: 16 rows 147 -> 134, 128 rows 182 -> 162, 256 rows 230 -> 217, uneven T = 1024 152 ->
+// 139 (on every item they cost 4% where experts have several tiles: T = 2731 215 -> 225).
 // Not faster: 4 x 2 waves holding the token fragments (24 x 256 rows 236 us), 8 waves each
 // with its own 32 weight rows loaded straight into registers (half-line loads: 289 us).
 //
@@ -565,7 +570,7 @@ __device__ __forceinline__ void store_c_hilo(const v4f (&acc)[8][4], float* xch,
 //   B   41 .. 144 rows  3 stages of 18 KB + 32 KB
 //   C    1 ..  40 rows  4 stages of  5 KB + 32 KB
 // (the rows at which the next deeper ring just fits into 160 KB beside the epilogue's and
-// the items' 9 KB)
+// the items' 7 KB)
 template <int NS, int ROWS, int NT>
 struct Gemm1Class {
     static constexpr int kNS = NS;                     // stages
@@ -580,6 +585,11 @@ struct Gemm1Class {
 };
 // mode bits of gemm1_prefill8_kernel
 constexpr int kPrefillRanked = 1, kPrefillThroughF16 = 2;
+// Largest T whose weights of one-tile experts are loaded non-temporal: whole calls over four
+// routings each were 6% faster for it at T = 800 .. 1400, 4% at 2000, 1% at 2731, and 0.7%
+// slower at 3500, where most weights belong to experts of several tiles.  The kernel for
+// larger T is compiled without the second set of K loops, which alone cost it 0.7%.
+constexpr int kOnceMaxT = 2560;
 
 using Gemm1A = Gemm1Class<2, 256, 4>;
 using Gemm1B = Gemm1Class<3, 144, 3>;
@@ -589,8 +599,10 @@ struct Gemm1Item {   // uniform part of an item; the per-lane DMA offsets live a
     const uint8_t* w;    // the expert's W1 from the item's first gate row on
     uint32_t wbytes;
     int row0, nrows, ng;
+    bool once;           // weights loaded non-temporal: the expert has no other row tile
 };
 
+template <bool ONCE>
 __global__ __launch_bounds__(512, 1) void gemm1_prefill8_kernel(
     const uint8_t* __restrict__ hidden, TokenScales sa, int T,
     const uint8_t* __restrict__ w1, const float* __restrict__ s1,
@@ -598,15 +610,17 @@ __global__ __launch_bounds__(512, 1) void gemm1_prefill8_kernel(
     const int* __restrict__ exp_off, const int* __restrict__ sorted_tok, Intermediate C, int mode) {
     constexpr int BM = 256;
     constexpr int NG = kI / 128;
-    constexpr int kItemCap = 64;                // per-workgroup item table
+    constexpr int kItemCap = 56;                // per-workgroup item table
     constexpr int kPool = std::max({Gemm1A::kBytes, Gemm1B::kBytes, Gemm1C::kBytes});
-    constexpr int kXch = kPool, kTokIds = kXch + 4 * BM * 4, kWsc = kTokIds + BM * 4, kItems = kWsc + 2 * 512;
+    constexpr int kXch = kPool, kTokIds = kXch + 4 * BM * 4, kWsc = kTokIds + BM * 4, kItems = kWsc + 2 * 512,
+                  kRows = kItems + kItemCap * (int)sizeof(int4);
     // one LDS object: the stages, the row-maximum exchange, the next item's tokens, two
-    // items' weight scales, the item table
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[kItems + kItemCap * sizeof(int4)];
+    // items' weight scales, the item table, the experts' rows
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[kRows + kEL * 4];
     static_assert(sizeof(lds) <= 160 * 1024, "LDS of a CU");
     int4* const s_items = reinterpret_cast<int4*>(lds + kItems);
     const int* const s_tok = reinterpret_cast<const int*>(lds + kTokIds);
+    int* const s_rows = reinterpret_cast<int*>(lds + kRows);
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
@@ -636,6 +650,7 @@ __global__ __launch_bounds__(512, 1) void gemm1_prefill8_kernel(
     int nr = (mode & kPrefillRanked) ? prefill_items_ranked<BM>(s_items, kItemCap, NG, base, G, exp_off, lds) : -1;
     if (nr < 0) nr = prefill_items<BM>(s_items, kItemCap, nitems, NG, base, G, tiles, exp_off);
     if (nr == 0) return;   // uniform: the whole workgroup has no item
+    if (ONCE && threadIdx.x < kEL) s_rows[threadIdx.x] = exp_off[threadIdx.x + 1] - exp_off[threadIdx.x];
     __syncthreads();
 
     // lane-dependent addresses that only the change of items needs are computed there, from a
@@ -667,6 +682,7 @@ __global__ __launch_bounds__(512, 1) void gemm1_prefill8_kernel(
         const size_t first = (size_t)m.x * kN1 + (size_t)it.ng * 128;
         it.w = w1 + first * kH;
         it.wbytes = (uint32_t)(((size_t)(m.x + 1) * kN1 - first) * kH);
+        it.once = ONCE && __builtin_amdgcn_readfirstlane(s_rows[m.x]) <= BM;
         return it;
     };
     // 8-row blocks of token rows this wave moves: NT wave + i (clamped into the class's rows,
@@ -692,12 +708,13 @@ __global__ __launch_bounds__(512, 1) void gemm1_prefill8_kernel(
     // K block kb of an item into a stage; past the last block the buffers have no bytes, so
     // that nothing moves and the number of loads in flight stays the same without a branch
     // in the K loop
-    auto issue_w = [&](auto cls, const Gemm1Item& it, int kb, int stage, int i0 = 0, int i1 = 4) {
+    auto issue_w = [&](auto cls, auto once, const Gemm1Item& it, int kb, int stage, int i0 = 0, int i1 = 4) {
         using Cl = decltype(cls);
         const __amdgpu_buffer_rsrc_t rs_w = buffer_rsrc(it.w, kb < kHB ? it.wbytes : 0u);
 #pragma unroll
         for (int i = i0; i < i1; ++i)
-            bdma16(rs_w, woff[i], (uint32_t)kb * kBlk, lds + stage * Cl::kW + (32 * wave + 8 * i) * kBlk);
+            bdma16<decltype(once)::value ? kNonTemporal : 0>(rs_w, woff[i], (uint32_t)kb * kBlk,
+                                                             lds + stage * Cl::kW + (32 * wave + 8 * i) * kBlk);
     };
     auto issue_t = [&](auto cls, int kb, int stage, int i0 = 0, int i1 = 5) {
         using Cl = decltype(cls);
@@ -715,7 +732,8 @@ __global__ __launch_bounds__(512, 1) void gemm1_prefill8_kernel(
         set_offsets(cls, it);
 #pragma unroll
         for (int k = 0; k < decltype(cls)::kNS; ++k) {
-            issue_w(cls, it, k, k);
+            if (ONCE && it.once) issue_w(cls, BoolC<ONCE>{}, it, k, k);
+            else issue_w(cls, BoolC<false>{}, it, k, k);
             if (decltype(cls)::kNS > 2 || k == 0) issue_t(cls, k, k);
             else issue_t(cls, k, k, 0, 2);   // the rest in the K loop
         }
@@ -743,7 +761,7 @@ __global__ __launch_bounds__(512, 1) void gemm1_prefill8_kernel(
         // NL: row blocks 128 wm + 16 j of this wave that are computed (the live ones, rounded
         // up to the instantiated counts; padding rows are computed on whatever the LDS holds
         // and never stored)
-        auto kloop = [&](auto cls, auto live) {
+        auto kloop_of = [&](auto cls, auto live, auto once) {
             using Cl = decltype(cls);
             constexpr int NL = decltype(live)::value;
             constexpr int NS = Cl::kNS;
@@ -772,8 +790,8 @@ __global__ __launch_bounds__(512, 1) void gemm1_prefill8_kernel(
             auto free_weights = [&](int kb, int stage) {
                 __builtin_amdgcn_sched_barrier(0);
                 lds_barrier();
-                if (NL > 4) issue_w(cls, cur, kb + NS, stage, 0, 1);
-                else issue_w(cls, cur, kb + NS, stage);
+                if (NL > 4) issue_w(cls, once, cur, kb + NS, stage, 0, 1);
+                else issue_w(cls, once, cur, kb + NS, stage);
                 __builtin_amdgcn_sched_barrier(0);
             };
             // every wave has read its last token fragment of K block kb, and block kb + 1 has
@@ -782,7 +800,7 @@ __global__ __launch_bounds__(512, 1) void gemm1_prefill8_kernel(
                 __builtin_amdgcn_sched_barrier(0);
                 __builtin_amdgcn_s_waitcnt(vmcnt_imm(kEarly ? 4 : (NS - 2) * (4 + Cl::kNT + 1)));
                 lds_barrier();
-                if (!kEarly) issue_w(cls, cur, kb + NS, stage);
+                if (!kEarly) issue_w(cls, once, cur, kb + NS, stage);
                 issue_t(cls, kb + NS, stage, 0, kFirstT);
                 __builtin_amdgcn_sched_barrier(0);
             };
@@ -848,7 +866,7 @@ __global__ __launch_bounds__(512, 1) void gemm1_prefill8_kernel(
                         }
                         __builtin_amdgcn_sched_barrier(0);
                         if (kEarly && j == 0) issue_t(cls, kb - 1 + NS, pstage, 2, 5);
-                        if (kEarly && NL > 4 && j >= 1 && j <= 3) issue_w(cls, cur, kb + NS, stage, j, j + 1);
+                        if (kEarly && NL > 4 && j >= 1 && j <= 3) issue_w(cls, once, cur, kb + NS, stage, j, j + 1);
                         __builtin_amdgcn_sched_barrier(0);
                         fgp = sv * wg;
                         fup = sv * wu;
@@ -868,6 +886,10 @@ __global__ __launch_bounds__(512, 1) void gemm1_prefill8_kernel(
             }
         };
         const int live = min(8, max(0, (cur.nrows - 128 * wm + 15) >> 4));
+        auto kloop = [&](auto cls, auto n) {
+            if (ONCE && cur.once) kloop_of(cls, n, BoolC<ONCE>{});
+            else kloop_of(cls, n, BoolC<false>{});
+        };
         if (cur.nrows > Gemm1B::kRows) {
             if (live > 6) kloop(Gemm1A{}, IntC<8>{});
             else if (live > 4) kloop(Gemm1A{}, IntC<6>{});
@@ -999,11 +1021,16 @@ bool launch_gemm1(int variant, const uint8_t* hidden, const TokenScales& sa, int
                                stream, hidden, sa, T, w1, s1, tiles, num_tiles, sorted_tok, C, c_wide);
             return true;
         }
-        case 4:
-            launch_kernel(gemm1_prefill8_kernel, dim3(prefill_grid), dim3(512), 0, stream,
-                               hidden, sa, T, w1, s1, tiles, num_tiles, exp_off, sorted_tok, C,
-                               (ranked ? kPrefillRanked : 0) | (through_f16 ? kPrefillThroughF16 : 0));
+        case 4: {
+            const int mode = (ranked ? kPrefillRanked : 0) | (through_f16 ? kPrefillThroughF16 : 0);
+            if (T <= kOnceMaxT)
+                launch_kernel(gemm1_prefill8_kernel<true>, dim3(prefill_grid), dim3(512), 0, stream, hidden, sa, T,
+                                   w1, s1, tiles, num_tiles, exp_off, sorted_tok, C, mode);
+            else
+                launch_kernel(gemm1_prefill8_kernel<false>, dim3(prefill_grid), dim3(512), 0, stream, hidden, sa, T,
+                                   w1, s1, tiles, num_tiles, exp_off, sorted_tok, C, mode);
             return true;
+        }
         default: return false;
     }
 }

@@ -63,7 +63,7 @@ inline bool g2_hilo(int v) { return v == 5; }        // GEMM2 reads the hi/lo fo
 // sides measured (GEMM1 + conversion + GEMM2 and the rest, four routings each, us): T = 560
 // 206-233 token-sharing, 216-239 prefill; 700 231-253, 227-245; 850 244-274, 232-254; 1000
 // 250-292, 238-262; 1344 287-349, 246-277.  The bound above keeps the ranked order's tables
-// (kRankMaxGroups groups, the kernel's 64 rounds) from running out.
+// (kRankMaxGroups groups, the kernel's 56 rounds) from running out.
 constexpr int32_t kRowClassMinT = 700;
 constexpr int32_t kRowClassMaxT = 16384;
 

@@ -385,9 +385,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void* base, 
 typedef __attribute__((address_space(3))) void lds_void_t;
 
 // buffer_load_dwordx4 ... lds: lane L copies 16 bytes from voff + soff to LDS l + 16 L.
+// AUX: the cache policy, 0 or kNonTemporal (data read once by one CU).
+constexpr int kNonTemporal = 2;
+template <int AUX = 0>
 __device__ __forceinline__ void bdma16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff,
                                        void* l) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void_t*)l, 16, voff, soff, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void_t*)l, 16, voff, soff, 0, AUX);
 }
 
 // buffer_load_dword ... lds: lane L copies 4 bytes from voff + soff to LDS l + 4 L.
