@@ -221,8 +221,9 @@ int forward_impl(const moe_mi355_args& a, void* workspace, size_t ws_bytes, hipS
         ok = moe::launch_gemm2_combine(inter, a.gemm2_weights, a.gemm2_weights_scale, tiles,
                                        num_tiles, meta, inv, sw, T, a.output, s);
     else if (ok && half)
-        ok = moe::launch_gemm2(plan.g2, inter, a.gemm2_weights, a.gemm2_weights_scale, tiles2,
-                               num_tiles2, meta, moe::dispatch_max_tiles(T, plan.tm2), rows, s);
+        ok = moe::launch_gemm2(T <= moe::host::kGemm2ClassMaxT ? 8 : plan.g2, inter, a.gemm2_weights,
+                               a.gemm2_weights_scale, tiles2, num_tiles2, meta,
+                               moe::dispatch_max_tiles(T, plan.tm2), rows, s);
     else if (ok)
         ok = moe::launch_gemm2(plan.g2, inter, a.gemm2_weights, a.gemm2_weights_scale, tiles,
                                num_tiles, meta, max_tiles, rows, s);

@@ -20,6 +20,7 @@
 // one e4m3 per element (kernel.cu:1086-1145), which does not meet atol = rtol = 1e-2
 // against the fp32 restatement; both forms used here do.
 
+#include "gemm2_rows.h"
 #include "gemm2_stream.h"
 
 MOE_STAMP_TABLE(gemm2)
@@ -284,66 +285,7 @@ __global__ __launch_bounds__(512, 1) void gemm2_prefill8_kernel(
         };
         with_live_blocks(live_blocks(64 * wm, cur.nrows), kloop);
 
-        // lane holds D[h = 64 wn + 16 n + 4 kq + v][row = 64 wm + 16 s + r16]
-        float mx = 0.f;
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-#pragma unroll
-            for (int n = 0; n < 4; ++n)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) mx = fmaxf(mx, fabsf(acc[s][n][v]));
-        if (!beyond_f16_in_wave(mx)) {
-            // the usual case: plain fp16, and the 4 zero exponents of a row's 64 columns
-            // as one 4-byte store (lane kq = 0 of the row).  The fp16 pairs of column
-            // blocks (0, 1) and (2, 3) are exchanged across the row's 4 lanes (lanes l,
-            // l+16, l+32, l+48: a 32-lane then a 16-lane swap) so that lane kq holds
-            // columns 8 kq .. 8 kq + 7 of the pair: one 16-byte store writes 64
-            // consecutive bytes of the row.
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const int rr = 64 * wm + 16 * s + r16;
-                uint32_t w[4][2];
-#pragma unroll
-                for (int n = 0; n < 4; ++n)
-#pragma unroll
-                    for (int q = 0; q < 2; ++q)
-                        w[n][q] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)acc[s][n][2 * q]) |
-                                  ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)acc[s][n][2 * q + 1]) << 16);
-#pragma unroll
-                for (int pr = 0; pr < 2; ++pr) {
-                    const int a = 2 * pr, b = 2 * pr + 1;
-#pragma unroll
-                    for (int q = 0; q < 2; ++q) {
-                        const auto p = __builtin_amdgcn_permlane32_swap(w[a][q], w[b][q], false, false);
-                        w[a][q] = p[0];
-                        w[b][q] = p[1];
-                    }
-#pragma unroll
-                    for (int q = 0; q < 2; ++q) {
-                        const auto p = __builtin_amdgcn_permlane16_swap(w[a][q], w[b][q], false, false);
-                        w[a][q] = p[0];
-                        w[b][q] = p[1];
-                    }
-                }
-                if (rr >= cur.nrows) continue;   // after the swaps: every lane takes part
-                const size_t row = (size_t)(cur.row0 + rr);
-                const int c0 = cur.hg * 256 + 64 * wn;
-#pragma unroll
-                for (int pr = 0; pr < 2; ++pr)
-                    *reinterpret_cast<v4u*>(rows.f16 + row * kH + c0 + 32 * pr + 8 * kq) =
-                        v4u{w[2 * pr][0], w[2 * pr][1], w[2 * pr + 1][0], w[2 * pr + 1][1]};
-                if (kq == 0) *reinterpret_cast<uint32_t*>(rows.exp + row * (kH / kGroup16) + c0 / kGroup16) = 0u;
-            }
-        } else {
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const int rr = 64 * wm + 16 * s + r16;
-#pragma unroll
-                for (int n = 0; n < 4; ++n)
-                    store_rows4(rows, rows_wide, cur.row0 + rr, cur.hg * 256 + 64 * wn + 16 * n + 4 * kq,
-                                acc[s][n], rr < cur.nrows);
-            }
-        }
+        store_prefill_rows(acc, rows, rows_wide, cur.row0, cur.nrows, cur.hg, wm, wn, r16, kq);
         cur = nxt;
     }
 }
@@ -369,6 +311,8 @@ static int grid_for2(long long work) { return (int)(work < 4096 ? work : 4096); 
 
 bool launch_gemm2_shared(const Intermediate&, int*, const uint8_t*, const float*, const int4*, const int*,
                          int, const ExpertRows&, hipStream_t);
+void launch_gemm2_class(const Intermediate&, int*, const uint8_t*, const float*, const int4*, const int*,
+                        const int*, const ExpertRows&, hipStream_t);
 
 // Variants (the tile height of the dispatch they expect, and the form of C they read):
 //   1  register-staged streaming, 32 columns x 1 row block per wave      16-row   fp16
@@ -377,6 +321,7 @@ bool launch_gemm2_shared(const Intermediate&, int*, const uint8_t*, const float*
 //      of the dispatch (whatever the first list's height)                         hi/lo
 //   7  token-sharing: 64-row tile x 128 columns, C rows shared in LDS (gemm2_shared.hip)
 //                                                                      64-row   fp16
+//   8  variant 5's tiles and sums by row classes (gemm2_class.hip)                    hi/lo
 bool launch_gemm2(int variant, const Intermediate& C, const uint8_t* w2, const float* s2,
                   const int4* tiles, const int* num_tiles, const int* exp_off, int max_tiles,
                   const ExpertRows& rows, hipStream_t stream) {
@@ -398,6 +343,9 @@ bool launch_gemm2(int variant, const Intermediate& C, const uint8_t* w2, const f
             return true;
         case 7:
             return launch_gemm2_shared(C, flags, w2, s2, tiles, num_tiles, max_tiles, rows, stream);
+        case 8:
+            launch_gemm2_class(C, flags, w2, s2, tiles, num_tiles, exp_off, rows, stream);
+            return true;
         default: return false;
     }
 }

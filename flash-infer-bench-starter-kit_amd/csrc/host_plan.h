@@ -67,6 +67,10 @@ inline bool g2_hilo(int v) { return v == 5; }        // GEMM2 reads the hi/lo fo
 constexpr int32_t kRowClassMinT = 700;
 constexpr int32_t kRowClassMaxT = 16384;
 
+// GEMM2 variant 5 runs by row classes (gemm2_class.hip, bit-identical rows) up to this T: the
+// whole call is 2.2 - 2.6% faster at T = 600, 800 and 1024, even at 1400 and 1.2% slower at 2000.
+constexpr int32_t kGemm2ClassMaxT = 1200;
+
 // The plan of a GEMM1 / GEMM2 pair, false when they cannot run together.  GEMM1
 // variant 5 is variant 1 with the dispatch folded in (T <= 64): every workgroup of a
 // persistent grid computes the call's dispatch from the routing ids, and the separate

@@ -1,8 +1,10 @@
 """The prefill GEMM1's row classes (how deep its operand rings run by the rows of an item)
 at their edges: experts with exactly the row counts where a 16-row block, a class (40 / 41,
-144 / 145) or a 256-row tile begins or ends, checked row by row against the fp32 oracle, and
+144 / 145) or a 256-row tile begins or ends, and where experts of one tile and of several
+share a call, checked row by row against the fp32 oracle, and
 pair 8/5 from T = 700 on, where this kernel stands in for the token-sharing GEMM1, against
-pair 7/5, whose C goes through fp16 and the conversion: bit-identical outputs."""
+pair 7/5, whose C goes through fp16 and the conversion: bit-identical outputs.  The GEMM2's row classes
+(T <= 1200) against the two-stage kernel of larger calls, bit-identical too."""
 import pytest
 import torch
 
@@ -13,7 +15,12 @@ pytestmark = pytest.mark.gpu
 
 EDGES = (1, 15, 16, 17, 32, 33, 39, 40, 41, 47, 48, 49, 64, 65, 127, 128, 129, 143, 144, 145,
          0, 160, 161, 239, 240, 241, 255, 256, 257, 0, 296, 397)
+# one-tile experts (weights loaded non-temporal up to T = 2560) among experts of several tiles
+MIXED = (1, 257, 0, 300, 256, 513, 41, 145) + (0,) * 23 + (17,)   # 1530 tokens
 SMALL = (1, 16, 17, 0, 40, 41, 64, 65, 128, 0, 129, 144, 145, 0, 64)   # 854 tokens
+
+# the GEMM2's classes (24 / 25, 64 / 65) and 128-row tiles, experts of one tile and of several
+GEMM2 = (24, 25, 64, 65, 128, 129, 1, 16, 17, 0, 32, 33, 48, 49, 0, 23, 63, 127, 257)   # 1101 tokens
 
 
 def _inputs(counts):
@@ -50,22 +57,23 @@ def _run(d, T, flags):
     return lay, ws, out
 
 
-@pytest.mark.parametrize("scales", ["gathered", "by token"])
-def test_row_counts_at_the_class_edges(scales):
+@pytest.mark.parametrize("counts,scales", [(EDGES, "gathered"), (EDGES, "by token"), (MIXED, "gathered")],
+                         ids=["gathered", "by token", "one-tile among larger"])
+def test_row_counts_at_the_class_edges(counts, scales):
     k = pkg("kernel")
     o = oracle()
-    d, T = _inputs(EDGES)
+    d, T = _inputs(counts)
     note(f"[gpu] row classes T={T} scales {scales}")
     lay, ws, _ = _run(d, T, k.FLAG_ROW_SCALES_OFF if scales == "by token" else 0)
     assert lay.tile_m == 256
     R = T * 8
     off = ws[lay.meta:lay.meta + 33 * 4].view(torch.int32).cpu().tolist()
-    assert [off[e + 1] - off[e] for e in range(32)] == list(EDGES)
+    assert [off[e + 1] - off[e] for e in range(32)] == list(counts)
     stok = ws[lay.sorted_tokens:lay.sorted_tokens + off[32] * 4].view(torch.int32).cpu().tolist()
     hi = ws[lay.intermediate:lay.intermediate + R * 2048].view(R, 2048)
     lo = ws[lay.intermediate + R * 2048:lay.intermediate + 2 * R * 2048].view(R, 2048)
     sc = ws[lay.intermediate_scales:lay.intermediate_scales + 16 * R * 4].view(torch.float32).view(16, R)
-    for e, n in enumerate(EDGES):
+    for e, n in enumerate(counts):
         # first, last and block- or tile-edge rows of the expert
         rows = sorted({off[e] + r for r in (0, 15, 16, 127, 128, 255, 256, n // 2, n - 1) if 0 <= r < n})
         if not rows:
@@ -90,3 +98,21 @@ def test_pair_8_5_is_bit_identical_to_7_5():
     for flags in (0, k.plan_flags(8, 5), k.FLAG_LIST_ORDER, k.FLAG_ROW_SCALES_OFF, k.FLAG_ROW_SCALES_ON):
         _, _, out = _run(d, T, flags)
         assert torch.equal(out.view(torch.int16), ref.view(torch.int16)), flags
+
+
+@pytest.mark.parametrize("pair", [(0, 0), (4, 5), (7, 5)], ids=["default", "4/5", "7/5"])
+def test_gemm2_classes_are_bit_identical_to_the_two_stage_kernel(pair):
+    """The same tokens in a call of more than 1200: an output row does not depend on the
+    call's other tokens, and there GEMM2 runs its two-stage kernel."""
+    k = pkg("kernel")
+    d, T = _inputs(GEMM2)
+    assert T <= 1200 < T + 200 <= 1344
+    note(f"[gpu] GEMM2 row classes T={T} pair {pair}")
+    flags = k.plan_flags(*pair) if pair[0] else 0
+    big = dict(d, output=torch.empty(T + 200, 7168, dtype=torch.bfloat16, device="cuda"))
+    for name in ("routing_logits", "hidden_states"):
+        big[name] = torch.cat([d[name].view(torch.uint8)] * 2)[:T + 200].view(d[name].dtype).contiguous()
+    big["hidden_states_scale"] = torch.cat([d["hidden_states_scale"]] * 2, dim=1)[:, :T + 200].contiguous()
+    _, _, out = _run(d, T, flags)
+    _, _, ref = _run(big, T + 200, flags)
+    assert torch.equal(out.view(torch.int16), ref[:T].view(torch.int16))
