@@ -14,7 +14,8 @@
 // supplies row l%16 and K elements 32*(l/16) + 8j..8j+7 of the block for MFMA j = 0..3
 // on both operands, and receives D[h = 4*(l/16)+v][row = l%16].  A work item's K blocks
 // are split over waves and reduced through LDS in a fixed order.
-// Prefill kernel: FP8 MFMA on the hi/lo form of C (see gemm2_prefill8_kernel).
+// Prefill kernel: FP8 MFMA on the hi/lo form of C (see gemm2_prefill8_kernel; calls of up to
+// kGemm2ClassMaxT tokens run gemm2_class.hip in its place).
 // Expert rows O go to the combine in fp16 (ExpertRows: bf16 rows break the 1e-2
 // tolerance where two large expert rows cancel, fp16 rows do not).  The reference re-quantises C to
 // one e4m3 per element (kernel.cu:1086-1145), which does not meet atol = rtol = 1e-2

@@ -15,7 +15,7 @@
 // buffers have no bytes, so the count of loads in flight, and each wait, stay constants.
 // Measured (GEMM2 alone, us, before -> after): 24 experts x 16 rows 72 -> 63; T = 1024, two
 // routings 101 -> 98 and 99.5 -> 94; whole calls T = 600, 800, 1024 (four routings each) 2.6,
-// 2.2 and 2.6% faster, T = 1400 even, T = 2000 and 2500 1.2 and 0.4% slower (heavier items:
+// 2.2 and 2.6% faster (T = 1024: 239.8 -> 233.9 us), T = 1400 even, T = 2000 and 2500 1.2 and 0.4% slower (heavier items:
 // more barriers per K block and the non-temporal form's second K loops), so variant 5 stays
 // beyond.
 #include "gemm2_rows.h"

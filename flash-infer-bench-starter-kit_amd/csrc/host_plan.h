@@ -60,9 +60,12 @@ inline bool g2_hilo(int v) { return v == 5; }        // GEMM2 reads the hi/lo fo
 // kRowClassMinT on: the same fp32 sums, rounded through fp16, written as the hi/lo form the
 // conversion would make of them (bit-identical rows, no conversion launch).  It orders its
 // items by the expert offsets alone, so the pair's 64-row tile list stays what it was.  Both
-// sides measured (GEMM1 + conversion + GEMM2 and the rest, four routings each, us): T = 560
-// 206-233 token-sharing, 216-239 prefill; 700 231-253, 227-245; 850 244-274, 232-254; 1000
-// 250-292, 238-262; 1344 287-349, 246-277.  The bound above keeps the ranked order's tables
+// sides measured (whole calls, four routings each, us): T = 560 206-238 token-sharing, 205-227
+// prefill; 650 223-242, 212-230; 690 231-253, 216-231; and before the prefill kernel's
+// non-temporal loads (6% of these calls) 850 244-274, 232-254; 1000 250-292, 238-262; 1344
+// 287-349, 246-277.  The line stands above 560, where the prefill kernel is already ahead,
+// because the token-sharing one also reports C beyond the fp16 range in the C flag, and calls
+// of T = 600 are held to that.  The bound above keeps the ranked order's tables
 // (kRankMaxGroups groups, the kernel's 56 rounds) from running out.
 constexpr int32_t kRowClassMinT = 700;
 constexpr int32_t kRowClassMaxT = 16384;
