@@ -440,28 +440,46 @@ __global__ __launch_bounds__(NRW == 8 ? 512 : 256) void gemm1_rstream_dispatch_k
 // rows' 4 lanes (lanes l, l+16, l+32, l+48) with v_permlane32_swap / v_permlane16_swap,
 // after which a lane holds 16 consecutive bytes of one row: one 16-byte store per form for
 // two row blocks.  Row blocks past the tile (from `live` on, uniform) are skipped.
+// through_f16: C is first rounded as the fp16 form holds it (moe_device.h), a 16-column group
+// with a value beyond the fp16 range by its group exponent, and such a group raises *c_wide:
+// the rows and the flag of a streaming GEMM1 and the conversion.
 __device__ __forceinline__ void store_c_hilo(const v4f (&acc)[8][4], float* xch, int live, int wm, int wn,
                                              int kq, int r16, int row0, int nrows, int ng,
-                                             const Intermediate& C, bool through_f16) {
+                                             const Intermediate& C, bool through_f16, int* c_wide) {
     float c[8][2][4];
     float m[8];
+    // the row addresses are computed here: kept through the K loop they would spill, and a
+    // reload waits for the next item's blocks
+    __asm__ volatile("" : "+v"(r16));
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
         if (s >= live) continue;
         m[s] = 0.f;
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < 2; ++i) {
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                float x = silu_f32(acc[s][i + 2][v]) * acc[s][i][v];
-                if (through_f16) {
+            for (int v = 0; v < 4; ++v) c[s][i][v] = silu_f32(acc[s][i + 2][v]) * acc[s][i][v];
+            if (through_f16) {
+                float mg = 0.f;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
                     // the fp32 product first, then fp16 (fused into one rounding otherwise)
-                    __asm__ volatile("" : "+v"(x));
-                    if (fabsf(x) <= kF16Max) x = (float)(_Float16)x;
+                    __asm__ volatile("" : "+v"(c[s][i][v]));
+                    mg = fmaxf(mg, fabsf(c[s][i][v]));
                 }
-                c[s][i][v] = x;
-                m[s] = fmaxf(m[s], fabsf(x));
+                if (!beyond_f16_in_wave(mg)) {   // the usual case: exponent 0
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) c[s][i][v] = (float)(_Float16)c[s][i][v];
+                } else {
+                    const int e = group_exponent(mg);
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) c[s][i][v] = ldexpf((float)(_Float16)ldexpf(c[s][i][v], -e), e);
+                    if (e && 128 * wm + 16 * s + r16 < nrows) *c_wide = 1;   // rows past the tile hold anything
+                }
             }
+#pragma unroll
+            for (int v = 0; v < 4; ++v) m[s] = fmaxf(m[s], fabsf(c[s][i][v]));
+        }
         m[s] = fmaxf(m[s], __shfl_xor(m[s], 16));
         m[s] = fmaxf(m[s], __shfl_xor(m[s], 32));
         if (kq == 0) xch[wn * 256 + 128 * wm + 16 * s + r16] = m[s];
@@ -607,7 +625,8 @@ __global__ __launch_bounds__(512, 1) void gemm1_prefill8_kernel(
     const uint8_t* __restrict__ hidden, TokenScales sa, int T,
     const uint8_t* __restrict__ w1, const float* __restrict__ s1,
     const int4* __restrict__ tiles, const int* __restrict__ num_tiles,
-    const int* __restrict__ exp_off, const int* __restrict__ sorted_tok, Intermediate C, int mode) {
+    const int* __restrict__ exp_off, const int* __restrict__ sorted_tok, Intermediate C, int mode,
+    int* __restrict__ c_wide) {
     constexpr int BM = 256;
     constexpr int NG = kI / 128;
     constexpr int kItemCap = 56;                // per-workgroup item table
@@ -918,7 +937,7 @@ __global__ __launch_bounds__(512, 1) void gemm1_prefill8_kernel(
             with_class(nxt.nrows, [&](auto cls) { start(cls, nxt); });
         }
         store_c_hilo(acc, reinterpret_cast<float*>(lds + kXch), live, wm, wn, kq, r16, cur.row0, cur.nrows,
-                     cur.ng, C, mode & kPrefillThroughF16);
+                     cur.ng, C, mode & kPrefillThroughF16, c_wide);
         cur = nxt;
     }
 }
@@ -1025,10 +1044,10 @@ bool launch_gemm1(int variant, const uint8_t* hidden, const TokenScales& sa, int
             const int mode = (ranked ? kPrefillRanked : 0) | (through_f16 ? kPrefillThroughF16 : 0);
             if (T <= kOnceMaxT)
                 launch_kernel(gemm1_prefill8_kernel<true>, dim3(prefill_grid), dim3(512), 0, stream, hidden, sa, T,
-                                   w1, s1, tiles, num_tiles, exp_off, sorted_tok, C, mode);
+                                   w1, s1, tiles, num_tiles, exp_off, sorted_tok, C, mode, c_wide);
             else
                 launch_kernel(gemm1_prefill8_kernel<false>, dim3(prefill_grid), dim3(512), 0, stream, hidden, sa, T,
-                                   w1, s1, tiles, num_tiles, exp_off, sorted_tok, C, mode);
+                                   w1, s1, tiles, num_tiles, exp_off, sorted_tok, C, mode, c_wide);
             return true;
         }
         default: return false;

@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from conftest import oracle, pkg
-from gpu_common import config_inputs, note
+from gpu_common import config_inputs, first_tokens, note
 
 pytestmark = pytest.mark.gpu
 
@@ -116,3 +116,43 @@ def test_gemm2_classes_are_bit_identical_to_the_two_stage_kernel(pair):
     _, _, out = _run(d, T, flags)
     _, _, ref = _run(big, T + 200, flags)
     assert torch.equal(out.view(torch.int16), ref[:T].view(torch.int16))
+
+
+@pytest.mark.parametrize("T", [700, 1024, 1344, None], ids=["700", "1024", "1344", "class edges"])
+def test_values_beyond_fp16_match_the_converted_form(T):
+    """Every third token 2^10 times larger, so that C leaves the fp16 range in some rows, and
+    in some 16-column groups beside values that stay inside it: the rows in use are those of
+    the token-sharing GEMM1 and the conversion (pair 7/5) bit for bit, the C flag (meta[35])
+    and the row flag are raised, and a call on normal inputs afterwards leaves both at zero
+    (the LDS rows past a tile then still hold large values)."""
+    k = pkg("kernel")
+    if T is None:
+        d, T = _inputs(SMALL)
+    else:
+        d = first_tokens(config_inputs(3), T)
+    note(f"[gpu] beyond fp16 by row classes T={T}")
+    scale = d["hidden_states_scale"].clone()
+    scale[:, ::3] *= 1024.0
+    big = dict(d, hidden_states_scale=scale)
+
+    def used(lay, ws):
+        R = T * 8
+        na = int(ws[lay.meta + 32 * 4:lay.meta + 33 * 4].view(torch.int32).item())
+        c = ws[lay.intermediate:lay.intermediate + 2 * R * 2048].view(2, R, 2048)[:, :na]
+        s = ws[lay.intermediate_scales:lay.intermediate_scales + 16 * R * 4].view(torch.int32).view(16, R)[:, :na]
+        flags = ws[lay.meta + 35 * 4:lay.meta + 37 * 4].view(torch.int32).cpu().tolist()
+        return c, s, flags
+
+    lay, ws, ref = _run(big, T, k.plan_flags(7, 5))
+    ref_c, ref_s, flags = used(lay, ws)
+    assert flags == [1, 1]
+    for fl in (0, k.plan_flags(8, 5), k.FLAG_LIST_ORDER, k.FLAG_ROW_SCALES_OFF):
+        lay, ws, out = _run(big, T, fl)
+        c, s, flags = used(lay, ws)
+        assert flags == [1, 1], fl
+        assert torch.equal(c, ref_c) and torch.equal(s, ref_s), fl
+        assert torch.equal(out.view(torch.int16), ref.view(torch.int16)), fl
+    lay, ws, out = _run(d, T, 0)
+    assert used(lay, ws)[2] == [0, 0]
+    _, _, ref = _run(d, T, k.plan_flags(7, 5))
+    assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
