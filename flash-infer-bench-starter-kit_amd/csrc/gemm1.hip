@@ -91,8 +91,8 @@ struct Gemm1Shared {
 
 // One item of gemm1_shared_kernel with CB live 16-row blocks (the tile has 16 CB - 15 ..
 // 16 CB rows): wave `wave` computes SwiGLU columns 16 ng .. 16 ng + 15 of rows row0 ..
-// row0 + nrows - 1.
-template <int D, int NWV, int CB>
+// row0 + nrows - 1.  AUX: the cache policy of the weight loads.
+template <int D, int NWV, int CB, int AUX>
 __device__ __forceinline__ void gemm1_shared_item(
     const uint8_t* __restrict__ hidden, const TokenScales& sa, __amdgpu_buffer_rsrc_t rs_h,
     __amdgpu_buffer_rsrc_t rs_s, const uint8_t* __restrict__ w1, const float* __restrict__ s1,
@@ -151,8 +151,8 @@ __device__ __forceinline__ void gemm1_shared_item(
     v4u bw[D][4];
     auto issue = [&](int kb, int ring) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)   // aux 2: nt, the weights are read once
-            bw[ring][i] = __builtin_amdgcn_raw_buffer_load_b128(rs_w, woff[i], (uint32_t)kb * kBlk, 2);
+        for (int i = 0; i < 4; ++i)
+            bw[ring][i] = __builtin_amdgcn_raw_buffer_load_b128(rs_w, woff[i], (uint32_t)kb * kBlk, AUX);
         uint8_t* st = tok0 + (kb % S::kStages) * S::kTokStage;
 #pragma unroll
         for (int i = 0; i < NT; ++i)
@@ -249,13 +249,21 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(WPE)))
     // token rows: T * 7168 < 2^32 (kMaxT); token scales: 56 x stride floats
     const __amdgpu_buffer_rsrc_t rs_h = buffer_rsrc(hidden, (uint32_t)T * kH);
     const __amdgpu_buffer_rsrc_t rs_s = buffer_rsrc(sa.p, (uint32_t)kHB * (uint32_t)sa.stride * 4);
-    // the first item's tile read before the tile count, both loads in flight together
-    // (blockIdx.x / kItems is inside the list's capacity: the grid has at most capacity x
-    // kItems workgroups; a workgroup past the count does not use what it read); each later
-    // tile is read after the item before it
-    const int4 tl0 = tiles[blockIdx.x / S::kItems];
+    // the first item's tile, and the expert of the tile before it, read before the tile count,
+    // all in flight together (blockIdx.x / kItems is inside the list's capacity: the grid has
+    // at most capacity x kItems workgroups; a workgroup past the count does not use what it
+    // read); each later tile is read after the item before it
+    const int t0 = blockIdx.x / S::kItems;
+    const int4 tl0 = tiles[t0];
+    const int pe0 = tiles[max(t0 - 1, 0)].x;
     int te = __builtin_amdgcn_readfirstlane(tl0.x), tr = __builtin_amdgcn_readfirstlane(tl0.y),
         tn = __builtin_amdgcn_readfirstlane(tl0.z);
+    // Weights of an expert with one tile are read once and loaded non-temporal; those of an
+    // expert with several are not, its tiles meet in L2 (a full tile counts as one of several).
+    // GEMM1, us, non-temporal on every item -> by this rule: T = 509 and four experts of 509 rows
+    // 214 -> 161, T = 400 and eight of 400 rows 243 -> 181, T = 600 and four of 600 270 -> 188,
+    // typical T = 509 130 -> 120, 300 136 -> 133.  Temporal on every item: 185, 181, 202, 141, 149.
+    bool several = tn == 64 || (t0 > 0 && __builtin_amdgcn_readfirstlane(pe0) == te);
     const int nwork = (*num_tiles) * S::kItems;
     int G = gridDim.x;
     if (WPE == 3 && G == 768 && nwork > 768 && nwork <= 1024) G = 512;
@@ -264,12 +272,19 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(WPE)))
         const int ng = (work % S::kItems) * NWV + wave;
         with_live_blocks(live_blocks(0, tn), [&](auto live) {
             constexpr int CB = decltype(live)::value;
-            if constexpr (CB > 0)
-                gemm1_shared_item<D, NWV, CB>(hidden, sa, rs_h, rs_s, w1, s1, te, tr, tn, ng,
-                                         sorted_tok, C, c_wide, lds, wave);
+            auto item = [&](auto aux) {
+                gemm1_shared_item<D, NWV, CB, decltype(aux)::value>(hidden, sa, rs_h, rs_s, w1, s1, te, tr, tn,
+                                                                    ng, sorted_tok, C, c_wide, lds, wave);
+            };
+            if constexpr (CB > 0) {
+                if (several) item(IntC<0>{});
+                else item(IntC<kNonTemporal>{});
+            }
         });
         if (work + G < nwork) {
-            const int4 t = tiles[(work + G) / S::kItems];
+            const int ti = (work + G) / S::kItems;
+            const int4 t = tiles[ti];
+            several = t.z == 64 || tiles[max(ti - 1, 0)].x == t.x;
             te = t.x;
             tr = t.y;
             tn = t.z;

@@ -22,6 +22,10 @@ SMALL = (1, 16, 17, 0, 40, 41, 64, 65, 128, 0, 129, 144, 145, 0, 64)   # 854 tok
 # the GEMM2's classes (24 / 25, 64 / 65) and 128-row tiles, experts of one tile and of several
 GEMM2 = (24, 25, 64, 65, 128, 129, 1, 16, 17, 0, 32, 33, 48, 49, 0, 23, 63, 127, 257)   # 1101 tokens
 
+# the token-sharing GEMM1's 64-row tiles: experts of one tile (weights loaded non-temporal),
+# of a full one, of several, and a light one right after an expert of several
+TOKEN_SHARING = (64, 63, 65, 1, 0, 128, 48, 49, 0, 33, 16, 17, 32)   # 516 tokens
+
 
 def _inputs(counts):
     """One local expert per token, counts[e] tokens for local expert e in a shuffled order;
@@ -156,3 +160,31 @@ def test_values_beyond_fp16_match_the_converted_form(T):
     assert used(lay, ws)[2] == [0, 0]
     _, _, ref = _run(d, T, k.plan_flags(7, 5))
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+
+
+@pytest.mark.parametrize("pair", [(8, 7), (7, 7)], ids=["8/7", "7/7"])
+def test_token_sharing_tiles_match_oracle(pair):
+    k = pkg("kernel")
+    o = oracle()
+    d, T = _inputs(TOKEN_SHARING)
+    assert 200 <= T <= 559
+    note(f"[gpu] token-sharing tiles T={T} pair {pair}")
+    lay, ws, _ = _run(d, T, k.plan_flags(*pair))
+    assert lay.tile_m == 64 and lay.intermediate_format == 0
+    R = T * 8
+    off = ws[lay.meta:lay.meta + 33 * 4].view(torch.int32).cpu().tolist()
+    assert [off[e + 1] - off[e] for e in range(len(TOKEN_SHARING))] == list(TOKEN_SHARING)
+    stok = ws[lay.sorted_tokens:lay.sorted_tokens + off[32] * 4].view(torch.int32).cpu().tolist()
+    f16 = ws[lay.intermediate + 2 * R * 2048:lay.intermediate + 4 * R * 2048].view(torch.float16).view(R, 2048)
+    for e, n in enumerate(TOKEN_SHARING):
+        rows = sorted({off[e] + r for r in (0, 15, 16, 47, 48, 63, 64, n - 1) if 0 <= r < n})
+        if not rows:
+            continue
+        got = f16[torch.tensor(rows, device="cuda")].float().cpu()
+        ref = o.swiglu_rows(d["hidden_states"], d["hidden_states_scale"], d["gemm1_weights"],
+                            d["gemm1_weights_scale"], e, [stok[r] for r in rows])
+        # fp16 rounds to 2^-11 of a value; twice that, and 2^-12 of the row's 128-column
+        # maximum for the fp32 sums' order
+        bmax = ref.view(-1, 16, 128).abs().amax(dim=2).repeat_interleave(128, dim=1)
+        err = (got - ref).abs()
+        assert (err <= ref.abs() * 2.0 ** -10 + bmax * 2.0 ** -12).all(), (e, n, float(err.max()))
