@@ -126,12 +126,14 @@ __device__ __forceinline__ void gemm1_shared_item(
     // the NWV groups of a workgroup lie in one 128-column scale block
     const float* sg = s1 + (size_t)(le * kN1B + (ng >> 3)) * kHB;
     const float* su = sg + (size_t)kIB * kHB;
-    // token rows of the live blocks (16 CB stage rows, 8 per instruction, clamped into the
-    // tile), spread over the waves: wave w moves rows 8 (w + NWV i) ...  Every wave issues
-    // the same number of loads per K block whatever is live, so that the number of loads in
-    // flight is known at compile time: the loads it has no rows (or, but for wave 0, no
-    // scales) for get an offset past the buffer, which moves nothing.
-    constexpr int NT = (2 * CB + NWV - 1) / NWV;
+    // The 2 CB loads of the token rows of the live blocks (16 CB stage rows, 8 per instruction,
+    // clamped into the tile) and the load of their scales, spread over the waves: wave w issues
+    // loads w, w + NWV, ...  Every wave issues the same number per K block whatever is live, so
+    // that the number of loads in flight is known at compile time: past the last one it issues
+    // one whose offset lies past the buffer, which moves nothing but takes its turn: with a scale
+    // load from every wave, 18 experts of up to 16 rows took 92.5 instead of 88.5 us.
+    constexpr int NT = (2 * CB + 1 + NWV - 1) / NWV;
+    constexpr int kScaleI = 2 * CB / NWV, kScaleWave = 2 * CB % NWV;   // the scales' load
     constexpr uint32_t kNothing = 0xfffffff0u;
     uint32_t toff[NT];
 #pragma unroll
@@ -143,9 +145,9 @@ __device__ __forceinline__ void gemm1_shared_item(
     }
     const int sr = min(lane, nrows - 1);
     const uint32_t so = (uint32_t)(sa.by_row ? row0 + sr : sorted_tok[row0 + sr]) * 4;
-    const uint32_t soff = wave == 0 ? so : kNothing;
-    const int sdst = 64 * kBlk + (wave == 0 ? 0 : 64 * 4);   // the others' zeros land past the scales
-    constexpr int kVm = 4 + NT + 1;                          // loads per wave and K block
+    if (wave == kScaleWave) toff[kScaleI] = so;
+    const int sdst = 64 * kBlk + (wave == kScaleWave ? 0 : 64 * 4);   // the others' zeros land past the scales
+    constexpr int kVm = 4 + NT;                              // loads per wave and K block
 
     // K block kb: weights in ring slot kb % D, token rows in stage kb % (D + 1)
     v4u bw[D][4];
@@ -155,9 +157,12 @@ __device__ __forceinline__ void gemm1_shared_item(
             bw[ring][i] = __builtin_amdgcn_raw_buffer_load_b128(rs_w, woff[i], (uint32_t)kb * kBlk, AUX);
         uint8_t* st = tok0 + (kb % S::kStages) * S::kTokStage;
 #pragma unroll
-        for (int i = 0; i < NT; ++i)
-            bdma16(rs_h, toff[i], (uint32_t)kb * kBlk, st + 8 * (wave + NWV * i) * kBlk);
-        bdma4(rs_s, soff, (uint32_t)kb * sa.stride * 4, st + sdst);
+        for (int i = 0; i < NT; ++i) {
+            if (i == kScaleI && (kScaleWave == 0 || wave >= kScaleWave))
+                bdma4(rs_s, toff[i], (uint32_t)kb * sa.stride * 4, st + sdst);
+            else
+                bdma16(rs_h, toff[i], (uint32_t)kb * kBlk, st + 8 * (wave + NWV * i) * kBlk);
+        }
     };
 #pragma unroll
     for (int k = 0; k < D - 1; ++k) issue(k, k);
@@ -229,7 +234,7 @@ __device__ __forceinline__ void gemm1_shared_item(
 }
 
 // WPE: the waves per SIMD the register allocation is held to (1: the compiler's choice,
-// 172 registers, two workgroups per CU; 3: 153 registers, three).
+// 172 registers, two workgroups per CU; 3: 142 registers, three).
 // With three per CU the kernel chooses, from the call's tile count, how many of its 768
 // workgroups work: items are equal (an item streams 128 weight rows over all of K), so the
 // rounds decide the time, and 768 < items <= 1024 takes two rounds either way, where two
