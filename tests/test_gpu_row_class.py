@@ -188,3 +188,34 @@ def test_token_sharing_tiles_match_oracle(pair):
         bmax = ref.view(-1, 16, 128).abs().amax(dim=2).repeat_interleave(128, dim=1)
         err = (got - ref).abs()
         assert (err <= ref.abs() * 2.0 ** -10 + bmax * 2.0 ** -12).all(), (e, n, float(err.max()))
+
+
+@pytest.mark.parametrize("T", [27000, 32768], ids=["in the item table", "past the item table"])
+def test_many_rounds_of_items(T):
+    """Every route local: 8 T rows.  The prefill GEMM1 ranks up to 56 rounds of items per
+    workgroup (T = 27000: 54); beyond (T = 32768: 66) it takes them in list order and resolves
+    those past its table one by one.  An output row does not depend on the call's other tokens:
+    the first and last tokens equal those of calls of their own."""
+    k = pkg("kernel")
+    wl = pkg("workloads")
+    cfg = wl.Config("all_local", T, 0, hot_local_experts=tuple(range(32)), seed=20261111)
+    d = dict(config_inputs(4))
+    d.update(wl.make_activations(cfg, device="cuda"))
+    d["output"] = torch.empty(T, 7168, dtype=torch.bfloat16, device="cuda")
+    note(f"[gpu] rounds of items, all local T={T}")
+    lay, ws, out = _run(d, T, 0)
+    off = ws[lay.meta:lay.meta + 33 * 4].view(torch.int32).cpu().tolist()
+    items = 16 * sum((b - a + 255) // 256 for a, b in zip(off, off[1:]))
+    assert off[32] == 8 * T and (items > 56 * 256) == (T == 32768)
+    if T == 27000:
+        _, _, ref = _run(d, T, k.FLAG_LIST_ORDER)
+        assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+        return
+    del ws
+    for part in (slice(0, 1700), slice(T - 1700, T)):
+        p = dict(d, routing_logits=d["routing_logits"][part].contiguous(),
+                 hidden_states=d["hidden_states"][part].contiguous(),
+                 hidden_states_scale=d["hidden_states_scale"][:, part].contiguous(),
+                 output=torch.empty(1700, 7168, dtype=torch.bfloat16, device="cuda"))
+        _, _, ref = _run(p, 1700, 0)
+        assert torch.equal(out[part].view(torch.int16), ref.view(torch.int16))
