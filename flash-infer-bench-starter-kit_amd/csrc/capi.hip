@@ -96,8 +96,8 @@ Profiler g_prof;
 // on the current GPU comes from hipGetSymbolAddress, once per device (kept in
 // g_scratch_dev), and only that address reaches the kernels.  Every call on one GPU
 // shares the array: nothing in it needs to start at zero (the route kernel clears the
-// flag words, or GEMM1 variant 9 marks them with the call's own tag; dispatch writes
-// every offset, count and row the later kernels read),
+// flag words, or, where GEMM1 routes, GEMM2 checks a set one against C's exponents; dispatch
+// writes every offset, count and row the later kernels read),
 // and calls that overlap on one GPU (two streams) race on it.
 constexpr size_t kScratchBytes = workspace_regions(MOE_MI355_NOALLOC_MAX_TOKENS).total;
 static_assert(kScratchBytes <= (size_t)64 << 20, "keep the per-GPU scratch array modest");

@@ -621,9 +621,11 @@ __device__ __forceinline__ void store_c_hilo(const v4f (&acc)[8][4], float* xch,
 //     meet in L2.
 //   - Past the last K block the buffers have no bytes: the loads stay in the loop without a
 //     branch, move nothing, and the counted waits hold in the last blocks too.
-// Measured (GEMM1, before -> after): 24 experts of 16 rows 173 -> 146 us, of 128 rows 205 ->
-// 182, of 256 rows 241 -> 226, of 512 rows 329 -> 323; uneven routings of T = 2731 259 ->
-// 214, T = 8192 385 -> 366 (335 ranked), skewed T = 4096 577 -> 550.  The non-temporal loads
+// Measured (GEMM1 us, two stages whatever the rows -> now): 24 experts of 16 rows 174 -> 133, of
+// 48 184 -> 140, of 128 202 -> 176, of 256 237 -> 220, of 512 321 -> 304; typical routings T =
+// 1024 185 -> 140, 2731 195 -> 165, 8192 356 -> 326 and 367 -> 370, 14107 439 -> 381; skewed T =
+// 4096 531 -> 518 and 543 -> 550; every route local, T = 8192 1700 -> 1746, T = 27000 5459 ->
+// 5673 (its K loop takes the same 96 us, the change of items 1.4 us more).  The non-temporal loads
 // alone: 16 rows 147 -> 134, 128 rows 182 -> 162, 256 rows 230 -> 217, uneven T = 1024 152 ->
 // 139 (on every item they cost 4% where experts have several tiles: T = 2731 215 -> 225).
 // Not faster: 4 x 2 waves holding the token fragments (24 x 256 rows 236 us), 8 waves each

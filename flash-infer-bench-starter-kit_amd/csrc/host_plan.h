@@ -57,21 +57,25 @@ inline bool g1_hilo(int v) { return v == 4; }        // GEMM1 writes the hi/lo f
 inline bool g2_hilo(int v) { return v == 5; }        // GEMM2 reads the hi/lo form (7: fp16)
 
 // Pair 8/5 runs the prefill GEMM1 in the place of the token-sharing one from T =
-// kRowClassMinT on: the same fp32 sums, rounded through fp16, written as the hi/lo form the
-// conversion would make of them (bit-identical rows, no conversion launch).  It orders its
-// items by the expert offsets alone, so the pair's 64-row tile list stays what it was.  Both
-// sides measured (whole calls, four routings each, us): T = 560 206-238 token-sharing, 205-227
-// prefill; 650 223-242, 212-230; 690 231-253, 216-231; and before the prefill kernel's
-// non-temporal loads (6% of these calls) 850 244-274, 232-254; 1000 250-292, 238-262; 1344
-// 287-349, 246-277.  The line stands above 560, where the prefill kernel is already ahead,
-// because the token-sharing one also reports C beyond the fp16 range in the C flag, and calls
-// of T = 600 are held to that.  The bound above keeps the ranked order's tables
-// (kRankMaxGroups groups, the kernel's 56 rounds) from running out.
+// kRowClassMinT on: the same fp32 sums, rounded as the fp16 form holds them, written as the
+// hi/lo form the conversion would make of them (bit-identical rows and C flag, no conversion
+// launch).  It orders its items by the expert offsets alone, so the pair's 64-row tile list
+// stays what it was.  The line is where typical routings break even; token-sharing / prefill
+// time of whole calls, eight or nine typical routings each, geometric mean (range): T = 560 0.97
+// (0.90 .. 0.99), 600 0.97 (0.87 .. 1.03), 650 0.97 (0.88 .. 1.04), 690 0.98 (0.88 .. 1.06), 720
+// 1.00 (0.88 .. 1.11), 800 1.01 (0.90 .. 1.13), 900 1.03 (0.90 .. 1.14), 1000 1.06 (0.91 ..
+// 1.23), 1344 1.13 (0.97 .. 1.21).  The low ends are routings of 17 to 20 light experts (5-8% of
+// them), whose 128-column items just miss one round of the CUs; T alone cannot tell them.  Four
+// hot experts favour the prefill kernel throughout (560 1.16, 690 1.24, 1100 1.36).  The bound
+// above keeps the ranked order's tables (kRankMaxGroups groups, the kernel's 56 rounds) from
+// running out.
 constexpr int32_t kRowClassMinT = 700;
 constexpr int32_t kRowClassMaxT = 16384;
 
 // GEMM2 variant 5 runs by row classes (gemm2_class.hip, bit-identical rows) up to this T: the
 // whole call is 2.2 - 2.6% faster at T = 600, 800 and 1024, even at 1400 and 1.2% slower at 2000.
+// Skewed routings, whose 128-row tiles are full, are level: 16 calls of T = 560 .. 1200 with two,
+// four or eight hot experts, from 1.4% slower (eight, T = 560: 410 -> 416 us) to 5.8% faster.
 constexpr int32_t kGemm2ClassMaxT = 1200;
 
 // The plan of a GEMM1 / GEMM2 pair, false when they cannot run together.  GEMM1

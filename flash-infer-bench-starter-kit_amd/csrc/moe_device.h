@@ -157,9 +157,11 @@ __device__ __forceinline__ int4 prefill_item(const int4* tab, int cap, int r, in
                 __builtin_amdgcn_readfirstlane(m.z), __builtin_amdgcn_readfirstlane(m.w)};
 }
 
-// Ranked order of the same groups, the prefill GEMM1's default: against list order its
-// GEMM1 was 6-13% faster at T = 1400 .. 8192 (two routings each; T = 8192 365 -> 335 and 305
-// -> 266 us) and 0-7% at T = 9000 .. 18000, level on skewed routings.  The experts are ranked by rows (descending, ties by index), each expert's
+// Ranked order of the same groups, the prefill GEMM1's default up to kRankMaxGroups groups and
+// `cap` rounds.  GEMM1 in list order -> ranked, us: T = 2000 128 -> 119, T = 6000 358 -> 309, T =
+// 8192 377 -> 378 and 338 -> 333, T = 16384 473 -> 431, skewed T = 4096 575 -> 570 and 533 -> 529,
+// every route local at T = 8192 1762 -> 1760.  The experts are ranked by rows (descending,
+// ties by index), each expert's
 // groups staying together in list order, and round r gives slot p = base on even and
 // G - 1 - base on odd rounds the item r * G + p of that order: the first rounds take
 // the experts with the most rows (full tiles), the lighter ones fill the last rounds,
@@ -302,20 +304,6 @@ __device__ __forceinline__ void dma4(const void* g, void* l) {
 // lgkmcnt left at their maxima).
 __device__ __forceinline__ constexpr int vmcnt_imm(int v) {
     return (v & 15) | ((v >> 4) << 14) | (7 << 4) | (15 << 8);
-}
-
-// vmcnt immediate for v = 0 .. 24 (uniform v; the switch keeps every wait an immediate)
-__device__ __forceinline__ void wait_vm_upto24(int v) {
-    switch (v) {
-#define MOE_WAIT_CASE(n) case n: __builtin_amdgcn_s_waitcnt(vmcnt_imm(n)); break;
-        MOE_WAIT_CASE(1) MOE_WAIT_CASE(2) MOE_WAIT_CASE(3) MOE_WAIT_CASE(4) MOE_WAIT_CASE(5)
-        MOE_WAIT_CASE(6) MOE_WAIT_CASE(7) MOE_WAIT_CASE(8) MOE_WAIT_CASE(9) MOE_WAIT_CASE(10)
-        MOE_WAIT_CASE(11) MOE_WAIT_CASE(12) MOE_WAIT_CASE(13) MOE_WAIT_CASE(14) MOE_WAIT_CASE(15)
-        MOE_WAIT_CASE(16) MOE_WAIT_CASE(17) MOE_WAIT_CASE(18) MOE_WAIT_CASE(19) MOE_WAIT_CASE(20)
-        MOE_WAIT_CASE(21) MOE_WAIT_CASE(22) MOE_WAIT_CASE(23) MOE_WAIT_CASE(24)
-#undef MOE_WAIT_CASE
-        default: __builtin_amdgcn_s_waitcnt(vmcnt_imm(0)); break;
-    }
 }
 
 // Workgroup barrier that orders LDS only.  __syncthreads() is a release/acquire of all
