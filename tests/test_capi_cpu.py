@@ -224,9 +224,9 @@ def test_list_order_flag_is_known_and_keeps_the_plan():
 def test_layout_reports_the_forced_plan():
     k = pkg("kernel")
     assert k.workspace_layout(64).tile_m == 16 and k.workspace_layout(64).intermediate_format == 0
-    # 32-row streaming tiles up to T = 199, then the token-sharing GEMM1 on 64-row tiles
-    # (fp16 C for the token-sharing GEMM2 up to T = 559, C converted to the hi/lo form for
-    # the prefill GEMM2 beyond), then 256-row prefill tiles
+    # 32-row streaming tiles up to T = 199, then 64-row tiles (fp16 C for the token-sharing
+    # GEMM2 up to T = 559, C rounded to fp16 and in the hi/lo form for the prefill GEMM2
+    # beyond), then 256-row prefill tiles
     assert [k.workspace_layout(t).tile_m for t in (89, 199, 200, 559, 560, 1344, 1345)] == \
         [32, 32, 64, 64, 64, 64, 256]
     assert [k.workspace_layout(t).intermediate_format for t in (199, 200, 559, 560, 1344, 1345)] == \

@@ -107,13 +107,15 @@ def test_small_odd_batches(T):
     assert st["frac_within"] == 1.0, st
 
 
-@pytest.mark.parametrize("T", [88, 89, 199, 200, 559, 560, 640, 641, 960, 961, 1344, 1345])
+@pytest.mark.parametrize("T", [88, 89, 199, 200, 399, 400, 559, 560, 640, 641, 699, 700, 960, 961,
+                               1200, 1201, 1344, 1345, 2560, 2561])
 def test_plan_boundaries_match_oracle(T):
     """Token counts on both sides of every change of kernel plan (16-row streaming,
-    32-row streaming, the token-sharing GEMM1 on 64-row tiles with three and then two
-    workgroups per CU feeding the token-sharing GEMM2 and then the prefill GEMM2, 256-row
-    prefill tiles) and of the dispatch (one workgroup up to T = 640, count and place
-    kernels over 256-token chunks beyond)."""
+    32-row streaming, the token-sharing GEMM1 on 64-row tiles feeding the token-sharing GEMM2
+    and from T = 560 the prefill GEMM2 by row classes, the prefill GEMM1 in its place from
+    T = 700, the two-stage prefill GEMM2 from 1201, 256-row prefill tiles from 1345, no
+    non-temporal weights from 2561) and of the dispatch (from the route kernel's masks from
+    T = 400)."""
     d = first_tokens(config_inputs(3), T)
     note(f"[gpu] plan boundary T={T}")
     out = run_forward(d)
@@ -131,8 +133,8 @@ def test_plan_boundaries_match_oracle(T):
                                      (600, 8, 7), (1000, 7, 7), (300, 8, 7), (150, 8, 7),
                                      (37, 7, 7), (1500, 8, 7)])
 def test_every_gemm_variant_matches_oracle(T, g1, g2):
-    """Each GEMM1 / GEMM2 kernel variant (forced with the call's plan flags) stays
-    within the tolerance."""
+    """Each GEMM1 / GEMM2 pair (forced with the call's plan flags; 8/5 at T = 1500 runs the
+    prefill GEMM1 in variant 8's place) stays within the tolerance."""
     d = first_tokens(config_inputs(3), T)
     note(f"[gpu] variants g1={g1} g2={g2} T={T}")
     out = run_forward(d, flags=pkg("kernel").plan_flags(g1, g2))
@@ -163,15 +165,15 @@ def test_batch_sizes_between_plan_boundaries(T, offset):
 
 
 def test_concurrent_streams_match_serial():
-    """Five calls of different plans (T = 8: routing, dispatch-in-GEMM1 streaming; 64;
-    600: token-sharing GEMM1 at three workgroups per CU; 1024: at two; 2000: prefill),
-    each on its own stream and workspace, issued together three times so that their
+    """Six calls of different plans (T = 8: routing, dispatch-in-GEMM1 streaming; 64; 300:
+    both token-sharing GEMMs; 600: token-sharing GEMM1, conversion and the class GEMM2; 1024:
+    prefill GEMM1 and the class GEMM2; 2000: prefill), each on its own stream and workspace, issued together three times so that their
     kernels overlap on the device: every output equals the serial one bit for bit (the
     library keeps no per-call state outside the caller's workspace)."""
     k = pkg("kernel")
     wl = pkg("workloads")
     full = config_inputs(3)
-    Ts = [8, 64, 600, 1024, 2000]
+    Ts = [8, 64, 300, 600, 1024, 2000]
     ds = [first_tokens(full, T) for T in Ts]
     note("[gpu] concurrent streams: serial reference")
     ref = [run_forward(d) for d in ds]
@@ -242,13 +244,13 @@ def test_row_order_token_scales_change_nothing(T):
 
 @pytest.mark.parametrize("idx,T,g1,g2", [(3, 1500, 0, 0), (3, 3500, 0, 0), (4, 3500, 0, 0),
                                          (3, 700, 4, 5), (3, 300, 4, 5), (1, None, 4, 5),
-                                         (0, None, 4, 5), (3, 3501, 0, 0)])
+                                         (0, None, 4, 5), (3, 3501, 0, 0), (3, None, 0, 0),
+                                         (4, None, 0, 0)])
 def test_ranked_item_order_changes_nothing(idx, T, g1, g2):
-    """The prefill GEMM1's ranked item order (the default up to T = 3500: every case but
-    the last) and tile-list order (FLAG_LIST_ORDER) give bit-identical outputs over every
-    token.  Only which workgroup computes an item differs; the workspace is filled with
-    0xff (fp8 / fp16 NaN) before each call, so an item that either order computed never
-    would show as NaN."""
+    """The prefill GEMM1's ranked item order (the default) and tile-list order
+    (FLAG_LIST_ORDER) give bit-identical outputs over every token.  Only which workgroup
+    computes an item differs; the workspace is filled with 0xff (fp8 / fp16 NaN) before each
+    call, so an item that either order computed never would show as NaN."""
     d = config_inputs(idx) if T is None else first_tokens(config_inputs(idx), T)
     k = pkg("kernel")
     wl = pkg("workloads")
@@ -268,13 +270,15 @@ def test_ranked_item_order_changes_nothing(idx, T, g1, g2):
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
 
 
-@pytest.mark.parametrize("T,g1,g2", [(64, 0, 0), (600, 0, 0), (2049, 0, 0), (600, 7, 5), (1100, 0, 0)])
+@pytest.mark.parametrize("T,g1,g2", [(64, 0, 0), (600, 0, 0), (2049, 0, 0), (600, 7, 5), (1100, 0, 0),
+                                     (1100, 8, 7)])
 def test_all_local_routing_matches_oracle(T, g1, g2):
     """Every token routed to 8 local experts (bias +3 on all 32 local experts, so group 0
     always wins and holds the whole top 8): N_a = 8T rows, the most the row-tile list
     and the workspace are sized for, on the 16-row plan, the 64-row token-sharing plans
-    (three workgroups per CU at T = 600, two at T = 1100, and two forced at T = 600:
-    150 rows per expert, full and partial 64-row tiles) and the 256-row plan."""
+    (T = 600 with three and, forced, two workgroups per CU: 150 rows per expert, full and
+    partial 64-row tiles; T = 1100 with the token-sharing GEMM2), the prefill GEMM1 in the
+    token-sharing one's place (T = 1100) and the 256-row plan."""
     k = pkg("kernel")
     wl = pkg("workloads")
     cfg = wl.Config("all_local", T, 0, hot_local_experts=tuple(range(32)), seed=20261111)
