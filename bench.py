@@ -324,7 +324,7 @@ def measure_config(idx: int, a, k, wl, o, steps: int, warmup: int, quantizer: bo
         "ms_per_step": round(ms_per_step, 6),
         "dtype": {0: "fp8_e4m3 GEMM1 + fp16 GEMM2 (W2 widened exactly), fp32 accumulate",
                   1: "fp8_e4m3 GEMM1 + fp8 hi/lo GEMM2 (two FP8 MFMAs per product), fp32 accumulate",
-                  2: "fp8_e4m3 GEMM1 (fp16 C, converted to fp8 hi/lo) + fp8 hi/lo GEMM2, "
+                  2: "fp8_e4m3 GEMM1 (C rounded to fp16, then fp8 hi/lo) + fp8 hi/lo GEMM2, "
                      "fp32 accumulate"}[lay.intermediate_format],
         "plan": {"tile_m": lay.tile_m, "dispatch_in_gemm1": bool(lay.dispatch_in_gemm1),
                  "combine_in_gemm2": bool(lay.combine_in_gemm2)},

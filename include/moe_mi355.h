@@ -114,10 +114,12 @@ typedef struct moe_mi355_args {
  *                                  three or two by the call's tile count (the default
  *                                  for 200 <= T <= 1344; in pair 8/5 from T = 700 on the
  *                                  prefill kernel computes the same rows in its place,
- *                                  bit-identical, and writes the hi/lo form itself);
+ *                                  bit-identical with the same C flag, and writes the
+ *                                  hi/lo form itself);
  *                                  GEMM2: 1 streaming 16-row, 3 streaming 32-row,
  *                                  5 prefill on a second list of 128-row tiles (the
- *                                  default for 560 <= T), 7 streaming with shared C
+ *                                  default for 560 <= T; up to T = 1200 by row classes,
+ *                                  bit-identical), 7 streaming with shared C
  *                                  rows on the 64-row tiles of GEMM1 7 or 8 (the default
  *                                  for 200 <= T <= 559).  A pair that cannot run
  *                                  together, or an unknown variant, gives
@@ -137,16 +139,16 @@ typedef struct moe_mi355_args {
  *                                  C's group exponents (and clears a stale one).
  *   MOE_MI355_FLAG_ROW_SCALES_ON / _OFF  GEMM1 reads the token scales gathered into row
  *                                  order / straight by token (default: gathered from
- *                                  T = 512, except under GEMM1 variants 7 and 8, which gather
- *                                  them itself).  Bit-identical results either way.  GEMM1
+ *                                  T = 512, except under the token-sharing GEMM1, which
+ *                                  gathers them itself).  Bit-identical results either way.  GEMM1
  *                                  variants 5 and 9 read them by token: _ON selects the
  *                                  separate dispatch at T <= 64 (and is an error with
  *                                  variant 5 or 9 forced).
  *   MOE_MI355_FLAG_LIST_ORDER      the prefill GEMM1 (variant 4) takes its work items in
  *                                  tile-list order (by default it ranks them by expert
- *                                  rows, which balances the workgroups' loads); which workgroup computes an item
- *                                  is all that changes, so the output is bit-identical
- *                                  either way.
+ *                                  rows, which balances the workgroups' loads); which
+ *                                  workgroup computes an item is all that changes, so
+ *                                  the output is bit-identical either way.
  * Every variant meets the same tolerance; the flags change speed only. */
 #define MOE_MI355_FLAG_PROFILE 1
 #define MOE_MI355_FLAG_FORCE_PLAN 2
