@@ -234,7 +234,7 @@ __device__ __forceinline__ void gemm1_shared_item(
 }
 
 // WPE: the waves per SIMD the register allocation is held to (1: the compiler's choice,
-// 172 registers, two workgroups per CU; 3: 142 registers, three).
+// 175 registers, two workgroups per CU; 3: 145 registers, three).
 // With three per CU the kernel chooses, from the call's tile count, how many of its 768
 // workgroups work: items are equal (an item streams 128 weight rows over all of K), so the
 // rounds decide the time, and 768 < items <= 1024 takes two rounds either way, where two
@@ -242,6 +242,16 @@ __device__ __forceinline__ void gemm1_shared_item(
 // other 512 (two per CU, the workgroups being spread over the CUs in launch order) take
 // the items.  Otherwise all 768 work (fewer rounds).  Which workgroup computes an item
 // changes nothing in the result.
+// Weights are loaded non-temporal unless their expert has kNear tiles or more (over 128 rows),
+// whose tiles meet in L2.  GEMM1 us in passes over four layers' own weights and routings,
+// non-temporal on every item -> by this rule: T = 509 with four experts of 509 rows 241 -> 191,
+// T = 400 with eight of 400 242 -> 175, T = 600 with four of 600 265 -> 203, every route local at
+// T = 509 392 -> 311; typical T = 509 133, 147, 130, 115 -> 129, 138, 135, 115.  From two tiles on
+// (kNear 2) typical calls of T = 509 .. 650 are 2-3% slower, as a second tile is often a few
+// rows; from four or six on, T = 509 with every route local loses 6 and 10%.  Passes that repeat one
+// layer do not show this: its weights are then still in the last-level cache.
+constexpr int kNear = 3;
+
 template <int D, int NWV, int WPE>
 __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(WPE))) void gemm1_shared_kernel(
     const uint8_t* __restrict__ hidden, TokenScales sa, int T,
@@ -254,22 +264,27 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(WPE)))
     // token rows: T * 7168 < 2^32 (kMaxT); token scales: 56 x stride floats
     const __amdgpu_buffer_rsrc_t rs_h = buffer_rsrc(hidden, (uint32_t)T * kH);
     const __amdgpu_buffer_rsrc_t rs_s = buffer_rsrc(sa.p, (uint32_t)kHB * (uint32_t)sa.stride * 4);
-    // the first item's tile, and the expert of the tile before it, read before the tile count,
+    // the first item's tile, and the experts of the tiles around it, read before the tile count,
     // all in flight together (blockIdx.x / kItems is inside the list's capacity: the grid has
-    // at most capacity x kItems workgroups; a workgroup past the count does not use what it
-    // read); each later tile is read after the item before it
+    // at most capacity x kItems workgroups, and the list's region holds twice as many 16-row
+    // tiles; a workgroup past the count does not use what it read); each later tile is read
+    // after the item before it
+    const int lane = threadIdx.x & 63;
+    auto expert_near = [&](int t) { return tiles[max(t - (kNear - 1) + min(lane, 2 * kNear - 2), 0)].x; };
+    // the expert of tile t has kNear tiles or more: as many of the kNear - 1 tiles on either
+    // side and itself are its own
+    auto has_several = [&](int t, int e, int near, int ntiles) {
+        const int i = t - (kNear - 1) + lane;
+        return __popcll(__ballot(lane <= 2 * kNear - 2 && i >= 0 && i < ntiles && near == e)) >= kNear;
+    };
     const int t0 = blockIdx.x / S::kItems;
     const int4 tl0 = tiles[t0];
-    const int pe0 = tiles[max(t0 - 1, 0)].x;
+    const int near0 = expert_near(t0);
     int te = __builtin_amdgcn_readfirstlane(tl0.x), tr = __builtin_amdgcn_readfirstlane(tl0.y),
         tn = __builtin_amdgcn_readfirstlane(tl0.z);
-    // Weights of an expert with one tile are read once and loaded non-temporal; those of an
-    // expert with several are not, its tiles meet in L2 (a full tile counts as one of several).
-    // GEMM1, us, non-temporal on every item -> by this rule: T = 509 and four experts of 509 rows
-    // 214 -> 161, T = 400 and eight of 400 rows 243 -> 181, T = 600 and four of 600 270 -> 188,
-    // typical T = 509 130 -> 120, 300 136 -> 133.  Temporal on every item: 185, 181, 202, 141, 149.
-    bool several = tn == 64 || (t0 > 0 && __builtin_amdgcn_readfirstlane(pe0) == te);
-    const int nwork = (*num_tiles) * S::kItems;
+    const int ntiles = *num_tiles;
+    const int nwork = ntiles * S::kItems;
+    bool several = has_several(t0, te, near0, ntiles);
     int G = gridDim.x;
     if (WPE == 3 && G == 768 && nwork > 768 && nwork <= 1024) G = 512;
     if ((int)blockIdx.x >= G) return;   // uniform: the whole workgroup
@@ -289,10 +304,11 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(WPE)))
         if (work + G < nwork) {
             const int ti = (work + G) / S::kItems;
             const int4 t = tiles[ti];
-            several = t.z == 64 || tiles[max(ti - 1, 0)].x == t.x;
+            const int near = expert_near(ti);
             te = t.x;
             tr = t.y;
             tn = t.z;
+            several = has_several(ti, te, near, ntiles);
         }
         __syncthreads();   // the next item's first loads reuse the token stages
     }

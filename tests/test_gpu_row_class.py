@@ -22,9 +22,9 @@ SMALL = (1, 16, 17, 0, 40, 41, 64, 65, 128, 0, 129, 144, 145, 0, 64)   # 854 tok
 # the GEMM2's classes (24 / 25, 64 / 65) and 128-row tiles, experts of one tile and of several
 GEMM2 = (24, 25, 64, 65, 128, 129, 1, 16, 17, 0, 32, 33, 48, 49, 0, 23, 63, 127, 257)   # 1101 tokens
 
-# the token-sharing GEMM1's 64-row tiles: experts of one tile (weights loaded non-temporal),
-# of a full one, of several, and a light one right after an expert of several
-TOKEN_SHARING = (64, 63, 65, 1, 0, 128, 48, 49, 0, 33, 16, 17, 32)   # 516 tokens
+# the token-sharing GEMM1's 64-row tiles: experts of one tile and of two (weights loaded
+# non-temporal), of three and four (not), and light ones next to them
+TOKEN_SHARING = (64, 63, 65, 1, 0, 130, 193, 0, 16, 17)   # 549 tokens
 
 
 def _inputs(counts):
@@ -177,7 +177,7 @@ def test_token_sharing_tiles_match_oracle(pair):
     stok = ws[lay.sorted_tokens:lay.sorted_tokens + off[32] * 4].view(torch.int32).cpu().tolist()
     f16 = ws[lay.intermediate + 2 * R * 2048:lay.intermediate + 4 * R * 2048].view(torch.float16).view(R, 2048)
     for e, n in enumerate(TOKEN_SHARING):
-        rows = sorted({off[e] + r for r in (0, 15, 16, 47, 48, 63, 64, n - 1) if 0 <= r < n})
+        rows = sorted({off[e] + r for r in (0, 15, 16, 47, 48, 63, 64, 127, 128, 191, 192, n - 1) if 0 <= r < n})
         if not rows:
             continue
         got = f16[torch.tensor(rows, device="cuda")].float().cpu()
