@@ -1,8 +1,6 @@
 // cform.hip -- the fp16 SwiGLU rows of the streaming GEMM1 kernels converted to the
-// fp8 hi/lo form of the prefill GEMM2 kernels, for the plans that pair the two: by default
-// 560 <= T < 700, where the token-sharing GEMM1 is the faster GEMM1 on typical routings and
-// the prefill GEMM2 the faster GEMM2 (host_plan.h has both lines; moe_device.h, Intermediate,
-// both forms).
+// fp8 hi/lo form of the prefill GEMM2 kernels, for the forced plans that pair the two (GEMM1
+// 1, 2 or 7 with GEMM2 5, and 8 below T = 560); moe_device.h, Intermediate, has both forms.
 //
 // Per row and 128-column block, the arithmetic of the prefill GEMM1 epilogue
 // (gemm1.hip, store_c_hilo): s = amax/448 (1 for an all-zero block),

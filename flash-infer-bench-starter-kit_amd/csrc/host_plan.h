@@ -32,13 +32,12 @@ constexpr int kMinTileM = 16;           // smallest row tile; sizes the tile lis
 // to T = 88, 32-row tiles (GEMM1 with two column groups per wave, GEMM2 with two row
 // blocks per wave) beyond.  From T = 200 GEMM1 is the token-sharing kernel on 64-row
 // tiles (fewer requests per output once an expert has dozens of rows; variant 8, which
-// runs three or two workgroups per CU as the call's tile count makes best), feeding up to
-// T = 559 the token-sharing GEMM2 on the same tiles (variant 7: fp16 C, no conversion;
-// 1-13 us faster than the neighbouring pairs at T = 200 .. 560 over three routings) and
-// beyond the prefill GEMM2 (128-row tiles, FP8 MFMA on the hi/lo form), from T = 700 with
-// the prefill GEMM1 in its place (row_class); from T = 1345 both
-// GEMMs are the MFMA-bound prefill kernels on 256-row tiles (GEMM2 on the 128-row second
-// list).  The boundaries come from wall-clock sweeps of the pairs at T = 72 .. 2560 on
+// runs three or two workgroups per CU as the call's tile count makes best), feeding the
+// token-sharing GEMM2 on the same tiles (variant 7: fp16 C, no conversion; 1-13 us faster
+// than the neighbouring pairs at T = 200 .. 560 over three routings).  From T = 560 the
+// prefill GEMM1 runs in its place (row_class) and the prefill GEMM2 on a second list of
+// 128-row tiles (FP8 MFMA on the hi/lo form); from T = 1345 the first list has 256-row
+// tiles too.  The boundaries come from wall-clock sweeps of the pairs at T = 72 .. 2560 on
 // MI355X over routing seeds from light to heavy routing to the local experts.
 struct Plan {
     int tm;        // tile height of the first list
@@ -60,22 +59,22 @@ inline bool g2_hilo(int v) { return v == 5; }        // GEMM2 reads the hi/lo fo
 // kRowClassMinT on: the same fp32 sums, rounded as the fp16 form holds them, written as the
 // hi/lo form the conversion would make of them (bit-identical rows and C flag, no conversion
 // launch).  It orders its items by the expert offsets alone, so the pair's 64-row tile list
-// stays what it was.  The line is where typical routings break even; token-sharing / prefill
-// time of whole calls, eight or nine typical routings each, geometric mean (range): T = 560 0.97
-// (0.90 .. 0.99), 600 0.97 (0.87 .. 1.03), 650 0.97 (0.88 .. 1.04), 690 0.98 (0.88 .. 1.06), 720
-// 1.00 (0.88 .. 1.11), 800 1.01 (0.90 .. 1.13), 900 1.03 (0.90 .. 1.14), 1000 1.06 (0.91 ..
-// 1.23), 1344 1.13 (0.97 .. 1.21).  The low ends are routings of 17 to 20 light experts (5-8% of
-// them), whose 128-column items just miss one round of the CUs; T alone cannot tell them.  Four
-// hot experts favour the prefill kernel throughout (560 1.16, 690 1.24, 1100 1.36).  The bound
-// above keeps the ranked order's tables (kRankMaxGroups groups, the kernel's 56 rounds) from
-// running out.
-constexpr int32_t kRowClassMinT = 700;
+// stays what it was.  The line is the pair's own lower end, where the two break even on typical
+// routings.  Token-sharing / prefill time of passes over four layers (own weights and
+// routings), four sets, geometric mean (range): T = 560 1.02 (0.98 .. 1.04), 600 1.03 (0.99 ..
+// 1.07), 650 1.05 (0.99 .. 1.09), 690 1.07 (1.00 .. 1.11), 800 1.10, 1000 1.15, 1344 1.17; four hot
+// experts 560 1.17, 690 1.23, 1000 1.20, 1344 1.30.  Single layers of about 25 light experts
+// (up to 80 rows) lose up to 8% at 560, 7% at 690 and 3% at 800, as the partial second round of
+// 128-column items holds them up; T alone cannot tell them.  The bound above keeps the ranked
+// order's tables (kRankMaxGroups groups, the kernel's 56 rounds) from running out.
+constexpr int32_t kRowClassMinT = 560;
 constexpr int32_t kRowClassMaxT = 16384;
 
-// GEMM2 variant 5 runs by row classes (gemm2_class.hip, bit-identical rows) up to this T: the
-// whole call is 2.2 - 2.6% faster at T = 600, 800 and 1024, even at 1400 and 1.2% slower at 2000.
-// Skewed routings, whose 128-row tiles are full, are level: 16 calls of T = 560 .. 1200 with two,
-// four or eight hot experts, from 1.4% slower (eight, T = 560: 410 -> 416 us) to 5.8% faster.
+// GEMM2 variant 5 runs by row classes (gemm2_class.hip, bit-identical rows) up to this T.  Passes
+// over four layers with typical routings, three sets each, are 1.3 .. 2.7% faster for it at T =
+// 560, 2.0 .. 3.4% at 650, 1.0 .. 2.5% at 800, 0.6 .. 2.5% at 1000, -0.9 .. 0.5% at 1200; one layer
+// at 2000 is 1.2% slower.  Skewed routings, whose 128-row tiles are full: 0.7% faster to 1.3%
+// slower (eight hot experts, T = 1000).
 constexpr int32_t kGemm2ClassMaxT = 1200;
 
 // The plan of a GEMM1 / GEMM2 pair, false when they cannot run together.  GEMM1

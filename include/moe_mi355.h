@@ -112,7 +112,7 @@ typedef struct moe_mi355_args {
  *                                  (pairs with GEMM2 5 and 7 only), two workgroups per
  *                                  CU, 8 the same held to three per CU, of which it runs
  *                                  three or two by the call's tile count (the default
- *                                  for 200 <= T <= 1344; in pair 8/5 from T = 700 on the
+ *                                  for 200 <= T <= 1344; in pair 8/5 from T = 560 on the
  *                                  prefill kernel computes the same rows in its place,
  *                                  bit-identical with the same C flag, and writes the
  *                                  hi/lo form itself);
@@ -267,7 +267,7 @@ typedef struct moe_mi355_workspace_layout {
                                   beyond the fp16 range (meta[35] set).
                                intermediate_format: 0 fp16 form, 1 hi/lo form, 2 fp16
                                form converted to the hi/lo form before GEMM2 (pair
-                               8/5 from T = 700 on writes those hi/lo rows directly,
+                               8/5 from T = 560 on writes those hi/lo rows directly,
                                and no fp16 form) */
     size_t intermediate_scales; /* fp32 [16, 8T]: s of row r, 128-column block b at [b][r] */
     size_t expert_out;      /* fp16  [8T, 7168]  GEMM2 output rows */

@@ -5,7 +5,7 @@ decides on the device, from the call's tile count, whether three or two workgrou
 work: two when the items (64-row tiles x 32) fall in (768, 1024], where both take two
 rounds, three otherwise.  The light routing of config 2 (707 rows) lands in that window,
 the heavy one (eight hot local experts, every token routed to them) far above it, so both
-paths run.  Every pair that can run at this T -- the default (8/5, which from T = 700 on
+paths run.  Every pair that can run at this T -- the default (8/5, which from T = 560 on
 runs the prefill GEMM1 by row classes over the same 64-row tile list), the two-per-CU
 token-sharing GEMM1 with the conversion (7/5), both token-sharing GEMM1s with the
 token-sharing GEMM2 (8/7, 7/7), the prefill pair (4/5) and the 32-row streaming GEMM1 with

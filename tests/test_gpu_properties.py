@@ -111,10 +111,10 @@ def test_small_odd_batches(T):
                                1200, 1201, 1344, 1345, 2560, 2561])
 def test_plan_boundaries_match_oracle(T):
     """Token counts on both sides of every change of kernel plan (16-row streaming,
-    32-row streaming, the token-sharing GEMM1 on 64-row tiles feeding the token-sharing GEMM2
-    and from T = 560 the prefill GEMM2 by row classes, the prefill GEMM1 in its place from
-    T = 700, the two-stage prefill GEMM2 from 1201, 256-row prefill tiles from 1345, no
-    non-temporal weights from 2561) and of the dispatch (from the route kernel's masks from
+    32-row streaming, the token-sharing GEMM1 on 64-row tiles feeding the token-sharing GEMM2,
+    from T = 560 the prefill GEMM1 in its place and the prefill GEMM2, both by row classes, the
+    two-stage prefill GEMM2 from 1201, 256-row prefill tiles from 1345, no non-temporal
+    weights from 2561) and of the dispatch (from the route kernel's masks from
     T = 400)."""
     d = first_tokens(config_inputs(3), T)
     note(f"[gpu] plan boundary T={T}")
@@ -129,12 +129,12 @@ def test_plan_boundaries_match_oracle(T):
 @pytest.mark.parametrize("T,g1,g2", [(64, 1, 1), (150, 1, 1), (64, 2, 3), (500, 2, 3),
                                      (1000, 4, 5), (3000, 4, 5), (1500, 2, 5), (150, 1, 5),
                                      (1000, 7, 5), (300, 7, 5), (37, 7, 5), (2000, 7, 5),
-                                     (600, 8, 5), (150, 8, 5), (1500, 8, 5), (500, 2, 5),
+                                     (600, 8, 5), (150, 8, 5), (500, 8, 5), (1500, 8, 5), (500, 2, 5),
                                      (600, 8, 7), (1000, 7, 7), (300, 8, 7), (150, 8, 7),
                                      (37, 7, 7), (1500, 8, 7)])
 def test_every_gemm_variant_matches_oracle(T, g1, g2):
-    """Each GEMM1 / GEMM2 pair (forced with the call's plan flags; 8/5 at T = 1500 runs the
-    prefill GEMM1 in variant 8's place) stays within the tolerance."""
+    """Each GEMM1 / GEMM2 pair (forced with the call's plan flags; 8/5 from T = 560 on runs
+    the prefill GEMM1 in variant 8's place) stays within the tolerance."""
     d = first_tokens(config_inputs(3), T)
     note(f"[gpu] variants g1={g1} g2={g2} T={T}")
     out = run_forward(d, flags=pkg("kernel").plan_flags(g1, g2))
@@ -166,8 +166,8 @@ def test_batch_sizes_between_plan_boundaries(T, offset):
 
 def test_concurrent_streams_match_serial():
     """Six calls of different plans (T = 8: routing, dispatch-in-GEMM1 streaming; 64; 300:
-    both token-sharing GEMMs; 600: token-sharing GEMM1, conversion and the class GEMM2; 1024:
-    prefill GEMM1 and the class GEMM2; 2000: prefill), each on its own stream and workspace, issued together three times so that their
+    both token-sharing GEMMs; 600 and 1024: prefill GEMM1 and the class GEMM2; 2000: prefill),
+    each on its own stream and workspace, issued together three times so that their
     kernels overlap on the device: every output equals the serial one bit for bit (the
     library keeps no per-call state outside the caller's workspace)."""
     k = pkg("kernel")
@@ -270,15 +270,15 @@ def test_ranked_item_order_changes_nothing(idx, T, g1, g2):
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
 
 
-@pytest.mark.parametrize("T,g1,g2", [(64, 0, 0), (600, 0, 0), (2049, 0, 0), (600, 7, 5), (1100, 0, 0),
+@pytest.mark.parametrize("T,g1,g2", [(64, 0, 0), (500, 0, 0), (600, 0, 0), (2049, 0, 0), (600, 7, 5), (1100, 0, 0),
                                      (1100, 8, 7)])
 def test_all_local_routing_matches_oracle(T, g1, g2):
     """Every token routed to 8 local experts (bias +3 on all 32 local experts, so group 0
     always wins and holds the whole top 8): N_a = 8T rows, the most the row-tile list
     and the workspace are sized for, on the 16-row plan, the 64-row token-sharing plans
-    (T = 600 with three and, forced, two workgroups per CU: 150 rows per expert, full and
-    partial 64-row tiles; T = 1100 with the token-sharing GEMM2), the prefill GEMM1 in the
-    token-sharing one's place (T = 1100) and the 256-row plan."""
+    (T = 500 by default and T = 1100 forced, with three workgroups per CU, T = 600 forced, with
+    two: 150 rows per expert, full and partial 64-row tiles), the prefill GEMM1 in the
+    token-sharing one's place (T = 600 and 1100 by default) and the 256-row plan."""
     k = pkg("kernel")
     wl = pkg("workloads")
     cfg = wl.Config("all_local", T, 0, hot_local_experts=tuple(range(32)), seed=20261111)
@@ -386,11 +386,14 @@ def test_values_beyond_fp16_range_32_row_streaming_plan():
     _huge_inputs_check(d, c_flag=1)
 
 
-def test_values_beyond_fp16_range_token_sharing_three_per_cu():
-    """T = 600 (the token-sharing GEMM1 at three workgroups per CU, the plan there)."""
-    d = first_tokens(config_inputs(3), 600)
-    note("[gpu] values beyond the fp16 range, T=600, GEMM1 variant 8")
-    _huge_inputs_check(d, c_flag=1)
+@pytest.mark.parametrize("T,g1,g2", [(600, 0, 0), (500, 8, 5), (500, 0, 0)])
+def test_values_beyond_fp16_range_token_sharing_three_per_cu(T, g1, g2):
+    """The token-sharing GEMM1 at three workgroups per CU: T = 500 by default (with the
+    token-sharing GEMM2) and with the conversion; and pair 8/5 at T = 600, where the prefill
+    GEMM1 stands in for it and raises the same flag."""
+    d = first_tokens(config_inputs(3), T)
+    note(f"[gpu] values beyond the fp16 range, T={T}, pair 8/5 or the default")
+    _huge_inputs_check(d, c_flag=1, flags=pkg("kernel").plan_flags(g1, g2) if g1 else 0)
 
 
 def test_values_beyond_fp16_range_token_sharing_gemm1():

@@ -2,7 +2,7 @@
 at their edges: experts with exactly the row counts where a 16-row block, a class (40 / 41,
 144 / 145) or a 256-row tile begins or ends, and where experts of one tile and of several
 share a call, checked row by row against the fp32 oracle, and
-pair 8/5 from T = 700 on, where this kernel stands in for the token-sharing GEMM1, against
+pair 8/5 from T = 560 on, where this kernel stands in for the token-sharing GEMM1, against
 pair 7/5, whose C goes through fp16 and the conversion: bit-identical outputs.  The GEMM2's row classes
 (T <= 1200) against the two-stage kernel of larger calls, bit-identical too."""
 import pytest
@@ -96,7 +96,7 @@ def test_row_counts_at_the_class_edges(counts, scales):
 def test_pair_8_5_is_bit_identical_to_7_5():
     k = pkg("kernel")
     d, T = _inputs(SMALL)
-    assert T >= 700
+    assert T >= 560
     note(f"[gpu] pair 8/5 by row classes T={T}")
     _, _, ref = _run(d, T, k.plan_flags(7, 5))
     for flags in (0, k.plan_flags(8, 5), k.FLAG_LIST_ORDER, k.FLAG_ROW_SCALES_OFF, k.FLAG_ROW_SCALES_ON):
@@ -122,7 +122,7 @@ def test_gemm2_classes_are_bit_identical_to_the_two_stage_kernel(pair):
     assert torch.equal(out.view(torch.int16), ref[:T].view(torch.int16))
 
 
-@pytest.mark.parametrize("T", [700, 1024, 1344, None], ids=["700", "1024", "1344", "class edges"])
+@pytest.mark.parametrize("T", [560, 700, 1024, 1344, None], ids=["560", "700", "1024", "1344", "class edges"])
 def test_values_beyond_fp16_match_the_converted_form(T):
     """Every third token 2^10 times larger, so that C leaves the fp16 range in some rows, and
     in some 16-column groups beside values that stay inside it: the rows in use are those of
